@@ -19,6 +19,7 @@
 #include "fh_iter.hpp"
 #include "fh_micro.hpp"
 #include "fh_pot.hpp"
+#include "fh_rt_launch.hpp"
 
 using fh::AxisPlan;
 using fh::CGState;
@@ -270,8 +271,10 @@ struct fh_plan {
   int band[3] = {0, 0, 0};
   double op_scale = 1.0;         // factor of the operator G A (not of the bare projection)
   // fused mixed CG: a batch of iterations captured once as a HIP graph, replayed per batch
-  hipGraphExec_t it_exec[9] = {};  // captured batches of 1, 2, 4, 8 fused iterations, by length
-  const void* it_key[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  // captured batches of 1, 2, 4, 8 fused iterations, by length, precision (0 fp64, 1 fp32) and the
+  // direction buffer that the batch starts from
+  hipGraphExec_t it_exec[9][2][2] = {};
+  const void* it_key[2][5] = {};  // buffers the captured batches were built for, by precision
   bool it_graph_off = false;     // capture failed on this plan: direct launches from then on
   bool use_graphs = true;        // fh_plan_use_graphs
   int last_graph_batches = 0;    // batches of the last solve replayed from the graph
@@ -282,6 +285,7 @@ struct fh_plan {
   fh_iterate_fn it_fn = nullptr; // host callback on the iterate every it_every iterations (0: off)
   void* it_user = nullptr;
   int it_every = 0;
+  fh::rt::Config rt[2];          // runtime-radix passes: [fp64, fp32]
   std::vector<int> res_kit;      // the log of the last solve: iteration counts and norms
   std::vector<double> res_norm;
 };
@@ -534,6 +538,145 @@ int launch_cols(fh_plan* pl, int mode, int axis, int nc, cpx<T>* data, const GPa
   return FH_OK;
 }
 
+// ---- runtime-radix passes (fh_rt.hpp): spectrum component-major -------------------------------
+
+template <typename T>
+const fh::rt::Config& rt_config(const fh_plan* pl) {
+  return pl->rt[sizeof(T) == 8 ? 0 : 1];
+}
+
+// Whether the operator of this plan runs on the runtime-radix passes in precision T.
+template <typename T>
+bool rt_on(const fh_plan* pl) {
+  return !pl->generic && rt_config<T>(pl).ok;
+}
+
+fh::rt::Launch rt_launch(const fh_plan* pl) { return fh::rt::Launch{pl->stream, pl->prof_t0, pl->prof_t1}; }
+
+int rt_result(hipError_t e, const char* what) {
+  if (e != hipSuccess) return fail(FH_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
+  return FH_OK;
+}
+
+// Forward contiguous-axis (plane) pass of nc components into `spec`. upd: the fused CG's direction
+// update (a.in, a.pout, a.r, a.xc, a.partial, a.bpart set by the caller).
+template <typename T>
+int rt_fwd(fh_plan* pl, fh::rt::FwdArgs<T>& a, int nc, bool upd) {
+  const fh::rt::Config& c = rt_config<T>(pl);
+  a.g = c.g;
+  a.g.nc = nc;
+  a.g.dnc = fh::rt::make_div(nc);
+  a.st = pl->st;
+  a.tw2 = twiddles<T>(pl, 2);
+  a.tw1 = twiddles<T>(pl, 1);
+  return rt_result(fh::rt::launch_fwd<T>(c, a, upd, c.nblk / c.g.nc * nc, rt_launch(pl)), "forward pass");
+}
+
+template <typename T>
+int rt_inv(fh_plan* pl, fh::rt::InvArgs<T>& a, int nc, int* nblocks) {
+  const fh::rt::Config& c = rt_config<T>(pl);
+  a.g = c.g;
+  a.g.nc = nc;
+  a.g.dnc = fh::rt::make_div(nc);
+  a.tw2 = twiddles<T>(pl, 2);
+  a.tw1 = twiddles<T>(pl, 1);
+  const unsigned nb = c.nblk / c.g.nc * nc;
+  if (a.epi && nb > pl->partial_cap) return fail(FH_ERR_STATE, "partial buffer too small");
+  if (nblocks) *nblocks = (int)nb;
+  return rt_result(fh::rt::launch_inv<T>(c, a, nb, rt_launch(pl)), "inverse pass");
+}
+
+// Strided pass: mode 0 / 1 the transform of nc single components along `axis`, mode 2 the projection
+// pass (all components, the plan's projection axis).
+template <typename T>
+int rt_cols(fh_plan* pl, int mode, int axis, int nc, const cpx<T>* src, cpx<T>* dst, const GParams* g,
+            const int* halt, const fh::CgFin* fin = nullptr) {
+  const fh::rt::Config& c = rt_config<T>(pl);
+  const bool proj_axis = axis == (pl->n0 > 1 ? 0 : 1);
+  fh::rt::ColArgs<T> a{};
+  a.src = src;
+  a.dst = dst;
+  a.n2h = pl->n2h;
+  a.dn2h = c.g.dn2h;
+  a.ax = proj_axis ? c.a0 : c.g.a1;
+  a.tw = twiddles<T>(pl, axis);
+  a.halt = halt;
+  if (fin) a.fin = *fin;
+  a.total = (long long)nc * pl->nh;
+  a.cs = (int)pl->nh;
+  int nthr;
+  size_t lds;
+  long long outer;
+  if (proj_axis) {
+    a.es = pl->n0 > 1 ? pl->n1 * pl->n2h : pl->n2h;
+    a.nf = a.es;
+    a.ostride = pl->nh;
+    outer = mode == 2 ? 1 : nc;
+    a.lf = mode == 2 ? c.lf : c.lp0;
+    a.tpp = mode == 2 ? c.tpp_g : c.tpp_0;
+    nthr = mode == 2 ? c.nthr_g : c.nthr_0;
+    lds = mode == 2 ? c.lds_g : c.lds_0;
+  } else {
+    a.es = pl->n2h;
+    a.nf = pl->n2h;
+    a.ostride = (long long)pl->n1 * pl->n2h;
+    outer = (long long)nc * pl->n0;
+    a.lf = c.lp1;
+    a.tpp = c.tpp_1;
+    nthr = c.nthr_1;
+    lds = c.lds_1;
+  }
+  if (mode == 2) a.g = *g;
+  const int ncf = mode == 2 ? nc : 1;
+  a.ntiles = (a.nf + (1 << a.lf) - 1) >> a.lf;
+  a.dP = fh::rt::make_div((long long)ncf << a.lf);
+  a.dtiles = fh::rt::make_div(a.ntiles);
+  const long long nb = outer * a.ntiles;
+  if (nb > 0x7fffffffLL || (mode != 2 && nb * a.ntiles >= (1LL << 32))) return fail(FH_ERR_UNSUPPORTED, "grid too large");
+  return rt_result(fh::rt::launch_cols<T>(nc, mode, a, (unsigned)nb, nthr, lds, rt_launch(pl)), "strided pass");
+}
+
+// The strided passes between k_fwd and k_inv of the operator; `fin` goes to the first of them.
+template <typename T>
+int rt_middle(fh_plan* pl, cpx<T>* spec, const GParams& g, const int* halt, const fh::CgFin* fin = nullptr) {
+  const int nc = pl->ncomp;
+  const bool axis1 = pl->n0 > 1 && !rt_config<T>(pl).g.plane;
+  if (axis1) RETCHK(rt_cols<T>(pl, 0, 1, nc, spec, spec, nullptr, halt, fin));
+  RETCHK(rt_cols<T>(pl, 2, pl->n0 > 1 ? 0 : 1, nc, spec, spec, &g, halt, axis1 ? nullptr : fin));
+  if (axis1) RETCHK(rt_cols<T>(pl, 1, 1, nc, spec, spec, nullptr, halt));
+  return FH_OK;
+}
+
+template <typename T>
+int rt_operator_front(fh_plan* pl, const T* x, int kind, const T* coef, const int* halt) {
+  cpx<T>* spec = reinterpret_cast<cpx<T>*>(pl->spec);
+  const GParams g = make_gparams(pl, (kind != fh::COEF_NONE ? pl->op_scale : 1.0) / (double)pl->n);
+  fh::rt::FwdArgs<T> a{};
+  a.in = x;
+  a.coef = coef;
+  a.kind = kind;
+  a.out = spec;
+  a.halt = halt;
+  RETCHK(rt_fwd<T>(pl, a, pl->ncomp, false));
+  return rt_middle<T>(pl, spec, g, halt);
+}
+
+// Inverse pass of the operator from the plan's spectrum, epilogue epi (see k_inv).
+template <typename T>
+int rt_operator_back(fh_plan* pl, T* out, int epi, const T* w, float* r32, fh::CGState* st, const int* halt, int* nb) {
+  fh::rt::InvArgs<T> a{};
+  a.in = reinterpret_cast<cpx<T>*>(pl->spec);
+  a.out = out;
+  a.scale = T(1);
+  a.epi = epi;
+  a.w = w;
+  a.r32 = r32;
+  a.partial = pl->partial;
+  a.st = st;
+  a.halt = halt;
+  return rt_inv<T>(pl, a, pl->ncomp, nb);
+}
+
 // y = F^-1 G F (A x); kind COEF_NONE gives the bare projection. With w != null the
 // last pass also writes per-workgroup partial sums of y.w into pl->partial.
 // rvec != null: x is the CG direction, updated in place to rvec + beta x before use.
@@ -542,6 +685,7 @@ int launch_cols(fh_plan* pl, int mode, int axis, int nc, cpx<T>* data, const GPa
 template <typename T>
 int run_operator_front(fh_plan* pl, const T* x, int kind, const T* coef, const int* halt, const T* rvec) {
   const int nc = pl->ncomp;
+  if (rt_on<T>(pl)) return rt_operator_front<T>(pl, x, kind, coef, halt);  // rvec is null there
   cpx<T>* spec = reinterpret_cast<cpx<T>*>(pl->spec);
   const GParams g = make_gparams(pl, (kind != fh::COEF_NONE ? pl->op_scale : 1.0) / (double)pl->n);
   RETCHK(launch_rows_fwd<T>(pl, nc, x, coef, kind, spec, halt, rvec));
@@ -559,6 +703,7 @@ template <typename T>
 int run_operator(fh_plan* pl, const T* x, T* y, int kind, const T* coef, const T* w, const int* halt,
                  int* nblocks_out, const T* rvec = nullptr) {
   RETCHK(run_operator_front<T>(pl, x, kind, coef, halt, rvec));
+  if (rt_on<T>(pl)) return rt_operator_back<T>(pl, y, w ? 1 : 0, w, nullptr, pl->st, halt, nblocks_out);
   cpx<T>* spec = reinterpret_cast<cpx<T>*>(pl->spec);
   RETCHK(launch_rows_inv<T>(pl, pl->ncomp, spec, y, T(1), w, pl->partial, halt, nblocks_out));
   return FH_OK;
@@ -572,6 +717,10 @@ int run_operator_residual(fh_plan* pl, const double* x, const double* b, double*
                           int* np) {
   RETCHK(run_operator_front<double>(pl, x, pl->coef_kind, reinterpret_cast<const double*>(pl->coef64), nullptr,
                                     nullptr));
+  if (rt_on<double>(pl)) {
+    *fused = true;
+    return rt_operator_back<double>(pl, nullptr, 3, b, r, pl->st, nullptr, np);
+  }
   cpx<double>* spec = reinterpret_cast<cpx<double>*>(pl->spec);
   *fused = false;
   if (!pl->generic) {
@@ -612,6 +761,7 @@ int grid_blocks(long long n, int per = 256, int cap = 2048) {
 // the caller's next residual overwrites); otherwise G c goes to c and a separate pass adds it.
 static int run_project_add(fh_plan* pl, double* c, double* x) {
   RETCHK(run_operator_front<double>(pl, c, fh::COEF_NONE, nullptr, nullptr, nullptr));
+  if (rt_on<double>(pl)) return rt_operator_back<double>(pl, x, 2, nullptr, nullptr, pl->st_add, nullptr, nullptr);
   cpx<double>* spec = reinterpret_cast<cpx<double>*>(pl->spec);
   if (!pl->generic) {
     fh::LaunchCtx cx = make_ctx<double>(pl);
@@ -718,6 +868,16 @@ static int matvec_impl(fh_plan* pl, int dtype, const void* x, void* y, bool with
 
 template <typename T>
 static int rfftn_impl(fh_plan* pl, int ncomp, const T* x, cpx<T>* xhat) {
+  if (rt_on<T>(pl)) {
+    // every component in one launch per pass: the passes' spectrum is the 'r' layout
+    fh::rt::FwdArgs<T> a{};
+    a.in = x;
+    a.kind = fh::COEF_NONE;
+    a.out = xhat;
+    RETCHK(rt_fwd<T>(pl, a, ncomp, false));
+    if (pl->n0 > 1 && !rt_config<T>(pl).g.plane) RETCHK(rt_cols<T>(pl, 0, 1, ncomp, xhat, xhat, nullptr, nullptr));
+    return rt_cols<T>(pl, 0, pl->n0 > 1 ? 0 : 1, ncomp, xhat, xhat, nullptr, nullptr);
+  }
   const GParams g = make_gparams(pl, 1.0, 1);
   for (int c = 0; c < ncomp; ++c) {
     cpx<T>* out = xhat + (size_t)c * pl->nh;
@@ -736,6 +896,20 @@ template <typename T>
 static int irfftn_impl(fh_plan* pl, int ncomp, const cpx<T>* xhat, T* x) {
   const GParams g = make_gparams(pl, 1.0, 1);
   cpx<T>* tmp = reinterpret_cast<cpx<T>*>(pl->spec);
+  if (rt_on<T>(pl)) {
+    // as many components at a time as the plan's spectrum holds; the first pass reads xhat
+    for (int c0 = 0; c0 < ncomp; c0 += pl->ncomp) {
+      const int m = std::min(pl->ncomp, ncomp - c0);
+      RETCHK(rt_cols<T>(pl, 1, pl->n0 > 1 ? 0 : 1, m, xhat + (size_t)c0 * pl->nh, tmp, nullptr, nullptr));
+      if (pl->n0 > 1 && !rt_config<T>(pl).g.plane) RETCHK(rt_cols<T>(pl, 1, 1, m, tmp, tmp, nullptr, nullptr));
+      fh::rt::InvArgs<T> a{};
+      a.in = tmp;
+      a.out = x + (size_t)c0 * pl->n;
+      a.scale = T(1.0 / (double)pl->n);
+      RETCHK(rt_inv<T>(pl, a, m, nullptr));
+    }
+    return FH_OK;
+  }
   for (int c = 0; c < ncomp; ++c) {
     HIPCHK(hipMemcpyAsync(tmp, xhat + (size_t)c * pl->nh, (size_t)pl->nh * sizeof(cpx<T>),
                           hipMemcpyDeviceToDevice, pl->stream));
@@ -784,10 +958,63 @@ static int ensure_hist(fh_plan* pl, int len) {
 // pl->partial[0..kDeferMax), the inverse pass's to pl->partial[kDeferMax..2 kDeferMax)).
 constexpr int kDeferMax = 2048;
 
+void drop_graphs(fh_plan* pl);
+
 // Deferred alpha/beta: at most 6 * kDeferMax grid rows (every fixed-length row pass has at least 6
 // rows per workgroup, so at most kDeferMax workgroups) and room for both partial runs.
+template <typename T>
 static bool defer_applies(const fh_plan* pl) {
+  if (rt_on<T>(pl)) return pl->defer_ok && rt_config<T>(pl).nblk <= kDeferMax && pl->partial_cap >= 2 * (size_t)kDeferMax;
   return pl->defer_ok && (long long)pl->n0 * pl->n1 <= 6LL * kDeferMax && pl->partial_cap >= 2 * (size_t)kDeferMax;
+}
+
+// One fused CG iteration on the runtime-radix passes (any coefficient kind, both precisions): three
+// launches on a 2-D grid or where the planes fit LDS, five otherwise, and the beta kernel unless it
+// is deferred. pin is the direction of the previous iteration, pout the new one (the same buffer for an
+// isotropic coefficient).
+template <typename T>
+static int enqueue_fused_rt(fh_plan* pl, T* xc, T* r, T* pin, T* pout, const T* coef) {
+  const int* halt = &pl->st->halt;
+  cpx<T>* spec = reinterpret_cast<cpx<T>*>(pl->spec);
+  const bool defer = pl->cg_defer;
+  double* part1 = pl->partial;
+  double* part2 = defer ? pl->partial + kDeferMax : pl->partial;
+  const int nb = (int)rt_config<T>(pl).nblk;
+  fh::rt::FwdArgs<T> f{};
+  f.in = pin;
+  f.pout = pout;
+  f.coef = coef;
+  f.kind = pl->coef_kind;
+  f.r = r;
+  f.xc = xc;
+  f.out = spec;
+  f.partial = part1;
+  f.halt = halt;
+  if (defer) {
+    f.bpart = part2;
+    f.bnp = nb;
+  }
+  RETCHK(rt_fwd<T>(pl, f, pl->ncomp, true));
+  const GParams g = make_gparams(pl, 1.0 / (double)pl->n);
+  const fh::CgFin fin{pl->st, part1, defer ? part2 : nullptr, nb, defer ? nb : 0};
+  RETCHK(rt_middle<T>(pl, spec, g, halt, &fin));
+  fh::rt::InvArgs<T> b{};
+  b.in = spec;
+  b.out = r;
+  b.scale = T(1);
+  b.epi = 2;
+  b.partial = part2;
+  b.st = pl->st;
+  b.defer_beta = defer ? 1 : 0;
+  b.halt = halt;
+  RETCHK(rt_inv<T>(pl, b, pl->ncomp, nullptr));
+  if (defer) {
+    pl->defer_nb2 = nb;
+  } else {
+    hipLaunchKernelGGL(fh::k_cg_beta, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, part2, nb);
+    HIPCHK(hipGetLastError());
+  }
+  return FH_OK;
 }
 
 // One fused fp32 CG iteration. With pl->cg_defer (small grids) alpha and beta have no kernels of
@@ -864,6 +1091,69 @@ static void enqueue_flush(fh_plan* pl) {
                        pl->defer_nb2);
 }
 
+// Vectors of a fused solve: the correction (or, in fp64, the iterate), the residual and the two
+// direction buffers (one and the same where the iteration updates the direction in place).
+template <typename T>
+struct FusedVecs {
+  T *xc, *r, *p[2];
+  const T* coef;
+};
+
+// A batch of `len` fused iterations, the first of them iteration number `kit`, and the flush of a
+// deferred beta. With `graph` the batch is captured once as a HIP graph (kernel nodes only) and
+// replayed: one launch per batch. *ok = false (nothing enqueued) where no fused kernels cover the plan.
+template <typename T>
+static int fused_batch(fh_plan* pl, const FusedVecs<T>& v, int kit, int len, bool graph, bool* ok) {
+  const int prec = sizeof(T) == 8 ? 0 : 1;
+  const int par = v.p[0] == v.p[1] ? 0 : kit & 1;
+  auto enqueue = [&](bool* all) -> int {
+    for (int k = 0; k < len; ++k) {
+      if (rt_on<T>(pl)) {
+        RETCHK(enqueue_fused_rt<T>(pl, v.xc, v.r, v.p[(par + k) & 1], v.p[(par + k + 1) & 1], v.coef));
+        continue;
+      }
+      bool covered = false;
+      if constexpr (sizeof(T) == 4) RETCHK(enqueue_fused_iteration(pl, v.xc, v.r, v.p[0], v.coef, &covered));
+      if (!covered) {
+        *all = false;
+        return FH_OK;
+      }
+    }
+    enqueue_flush(pl);
+    return FH_OK;
+  };
+  *ok = true;
+  const void* key[5] = {v.xc, v.r, v.p[0], v.coef, pl->spec};
+  if (std::memcmp(key, pl->it_key[prec], sizeof(key)) != 0) {
+    drop_graphs(pl);
+    std::memcpy(pl->it_key[prec], key, sizeof(key));
+  }
+  hipGraphExec_t& ex = pl->it_exec[len][prec][par];
+  if ((graph || ex) && pl->use_graphs && !pl->it_graph_off) {
+    if (!ex) {
+      hipGraph_t gr = nullptr;
+      bool all = true;
+      int rc = FH_OK;
+      if (hipStreamBeginCapture(pl->stream, hipStreamCaptureModeRelaxed) != hipSuccess) all = false;
+      if (all) rc = enqueue(&all);
+      const hipError_t ec = hipStreamEndCapture(pl->stream, &gr);
+      if (!(all && rc == FH_OK && ec == hipSuccess && gr &&
+            hipGraphInstantiate(&ex, gr, nullptr, nullptr, 0) == hipSuccess)) {
+        ex = nullptr;
+        pl->it_graph_off = true;  // capture not available here: enqueue the kernels directly
+      }
+      if (gr) (void)hipGraphDestroy(gr);
+      (void)hipGetLastError();
+    }
+    if (ex) {
+      HIPCHK(hipGraphLaunch(ex, pl->stream));
+      ++pl->last_graph_batches;
+      return FH_OK;
+    }
+  }
+  return enqueue(ok);
+}
+
 // One CG iteration in precision T on vectors (x, r, p, Ap); everything halts on st->halt.
 // The direction update p = r + beta p of the previous iteration happens inside the first
 // pass of the matvec (beta = 0 with p = r on the first iteration).
@@ -874,7 +1164,7 @@ static int enqueue_iteration(fh_plan* pl, T* x, T* r, T* p, T* Ap, const T* coef
   const long long nv = (long long)pl->ncomp * pl->n;
   const int* halt = &pl->st->halt;
   int nb = 0;
-  const bool fused = pl->coef_kind == fh::COEF_ISO;
+  const bool fused = pl->coef_kind == fh::COEF_ISO && !rt_on<T>(pl);
   if (!fused)
     hipLaunchKernelGGL((fh::k_cg_pupdate<T>), dim3(grid_blocks(nv)), dim3(256), 0, pl->stream, nv, p, r, pl->st);
   RETCHK(run_operator<T>(pl, p, Ap, pl->coef_kind, coef, p, halt, &nb, fused ? r : nullptr));
@@ -910,18 +1200,47 @@ static int enqueue_true_residual(fh_plan* pl, const double* b, const double* x, 
   return FH_OK;
 }
 
-// 1 if every value of x is +0 or -0 (the usual initial guess x0 = 0 of a solve).
-static int field_is_zero(fh_plan* pl, const double* x, bool* zero) {
+// Work memory of the fused fp64 solve: iterate, residual and one or two direction buffers.
+static size_t fused64_bytes(const fh_plan* pl) {
+  const size_t nvp = ((size_t)pl->ncomp * pl->n + 63) / 64 * 64;
+  return (pl->coef_kind == fh::COEF_ISO ? 3 : 4) * nvp * sizeof(double);
+}
+
+// What a solve decides before it starts, with one synchronisation: *zero = every value of x is +0 or
+// -0 (the usual initial guess); *fused64 = the fused iteration serves this fp64 solve. It takes <p, A p>
+// for <p, G(A p)>, which are equal for p in the range of G; the directions stay in that range when b
+// lies in it, as every right-hand side G(...) of the homogenization problem does. A b with a part
+// outside of it (above kRangeTol of its norm; rounding leaves about 1e-15) keeps the operator form, and
+// so do solves that need every iterate (residual log, callback).
+constexpr double kRangeTol = 1e-12;
+
+static int solve_start(fh_plan* pl, int mode, const double* b, const double* x, bool* zero, bool* fused64) {
   const long long nv = (long long)pl->ncomp * pl->n;
-  int* flag = reinterpret_cast<int*>(pl->partial);  // free at this point of a solve
+  const bool check = mode == FH_SOLVE_FP64 && rt_on<double>(pl) && pl->fused_cg && pl->op_scale == 1.0 &&
+                     pl->res_every == 0 && !pl->it_fn;
+  double* sums = pl->aux;
+  int* flag = reinterpret_cast<int*>(pl->aux + 2);
   HIPCHK(hipMemsetAsync(flag, 0, sizeof(int), pl->stream));
   hipLaunchKernelGGL(fh::micro::k_count_nonzero, dim3(grid_blocks(nv, 256, 4096)), dim3(256), 0, pl->stream, nv, x,
                      flag);
+  if (check) {
+    RETCHK(ensure_work(pl, fused64_bytes(pl)));
+    RETCHK(rt_operator_front<double>(pl, b, fh::COEF_NONE, nullptr, nullptr));
+    int nb = 0;
+    RETCHK(rt_operator_back<double>(pl, nullptr, 3, b, reinterpret_cast<float*>(pl->work), pl->st, nullptr, &nb));
+    hipLaunchKernelGGL(fh::k_sum_partials, dim3(1), dim3(256), 0, pl->stream, pl->partial, nb, 1.0, sums);
+    const int gb = grid_blocks(nv);
+    hipLaunchKernelGGL(fh::k_dot_partial<double>, dim3(gb), dim3(256), 0, pl->stream, nv, b, b, pl->partial);
+    hipLaunchKernelGGL(fh::k_sum_partials, dim3(1), dim3(256), 0, pl->stream, pl->partial, gb, 1.0, sums + 1);
+  }
   HIPCHK(hipGetLastError());
-  int h = 1;
-  HIPCHK(hipMemcpyAsync(&h, flag, sizeof(int), hipMemcpyDeviceToHost, pl->stream));
+  double h[3] = {0.0, 0.0, 0.0};
+  HIPCHK(hipMemcpyAsync(h, pl->aux, sizeof(h), hipMemcpyDeviceToHost, pl->stream));
   HIPCHK(hipStreamSynchronize(pl->stream));
-  *zero = h == 0;
+  int n = 1;
+  std::memcpy(&n, &h[2], sizeof(int));
+  *zero = n == 0;
+  *fused64 = check && std::sqrt(h[0]) <= kRangeTol * std::sqrt(h[1]);
   return FH_OK;
 }
 
@@ -1082,10 +1401,12 @@ int pot_operator(fh_plan* pl, cpx<T>* p, const cpx<T>* r, cpx<T>* out, T* re, co
 // plan's projection, band, kernel family and coefficient at capture time. Called by every entry
 // point that changes one of those (all entry points have finished their GPU work on return).
 void drop_graphs(fh_plan* pl) {
-  for (auto& e : pl->it_exec) {
-    if (e) (void)hipGraphExecDestroy(e);
-    e = nullptr;
-  }
+  for (auto& len : pl->it_exec)
+    for (auto& prec : len)
+      for (auto& e : prec) {
+        if (e) (void)hipGraphExecDestroy(e);
+        e = nullptr;
+      }
 }
 
 // Length of the next batch of CG iterations between two host synchronisations: the iterations
@@ -1114,6 +1435,45 @@ struct BatchPredictor {
     return std::min(len, cap);
   }
 };
+
+// The fp64 CG on fused iterations: the operations of the reference's CG with the solution update one
+// iteration late (inside the next forward pass) and <p, A p> formed there. s: the host copy of the CG
+// state, final on return.
+static int cg_fused64(fh_plan* pl, const double* b, double* x, bool x0_zero, CGState& s) {
+  const long long nv = (long long)pl->ncomp * pl->n;
+  const long long nvp = (nv + 63) / 64 * 64;  // 512-byte aligned sub-buffers
+  const bool two = pl->coef_kind != fh::COEF_ISO;
+  double* xw = (double*)pl->work;  // the plan's own iterate: captured batches keep its address
+  double* r = xw + nvp;
+  double* p0 = r + nvp;
+  const FusedVecs<double> v{xw, r, {p0, two ? p0 + nvp : p0}, pl->coef64};
+  pl->cg_defer = defer_applies<double>(pl);
+  pl->defer_nb2 = 0;
+  if (x0_zero) {
+    HIPCHK(hipMemsetAsync(xw, 0, (size_t)nv * sizeof(double), pl->stream));
+  } else {
+    HIPCHK(hipMemcpyAsync(xw, x, (size_t)nv * sizeof(double), hipMemcpyDeviceToDevice, pl->stream));
+  }
+  RETCHK(enqueue_true_residual<double>(pl, b, x, p0, r, x0_zero));
+  BatchPredictor pred;
+  int len = 8;
+  pl->last_graph_batches = 0;
+  for (int batch = 0;; ++batch) {
+    bool ok = true;
+    RETCHK(fused_batch<double>(pl, v, s.kit, len, batch > 0, &ok));
+    HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
+    HIPCHK(hipStreamSynchronize(pl->stream));
+    if (s.done) break;
+    len = pred.next(s, s.tol, 8);
+  }
+  const int gb = grid_blocks(nv);
+  if (s.pend)
+    hipLaunchKernelGGL(fh::k_fold_step, dim3(gb), dim3(256), 0, pl->stream, nv, xw, v.p[s.kit & 1], pl->st);
+  // x0 = 0: x <- G x once, removing the rounding outside the range of G (as the operator form)
+  if (x0_zero) return run_operator<double>(pl, xw, x, fh::COEF_NONE, nullptr, nullptr, nullptr, nullptr);
+  HIPCHK(hipMemcpyAsync(x, xw, (size_t)nv * sizeof(double), hipMemcpyDeviceToDevice, pl->stream));
+  return FH_OK;
+}
 
 }  // namespace
 
@@ -1273,8 +1633,22 @@ int fh_plan_create(int dim, const int* N, const double* Y, int physics, int prim
     }
     RowCfg rc32;
     row_config(pl->ax[2], pl->ncomp, sizeof(cpx<float>), (long long)pl->n0 * pl->n1, &rc32);
+    pl->rt[0] = fh::rt::make_config(sizeof(double), pl->n0, pl->n1, pl->n2, pl->ncomp);
+    pl->rt[1] = fh::rt::make_config(sizeof(float), pl->n0, pl->n1, pl->n2, pl->ncomp);
+    for (int i = 0; i < 2; ++i) {
+      // Where the fixed-length passes cover a 3-D grid, they stay the faster ones if the planes do not
+      // fit LDS (243^3: 329 against 395 us in single, 758 against 1060 us in double precision) and for
+      // double-precision planes of more than half of the LDS that need three stages an axis (125^3: 104
+      // against 112 us).
+      const fh::rt::Config& c = pl->rt[i];
+      const bool slow_plane = c.g.plane && c.lds > fh::rt::kLdsBytes / 2 && c.g.a2.nst > 2;
+      const bool fixed = pl->n0 > 1 && fh::fixed_length_supported(pl->n0) && fh::fixed_length_supported(pl->n1) &&
+                         fh::fixed_length_supported(pl->n2);
+      if (fixed && (!c.g.plane || slow_plane)) pl->rt[i].ok = false;
+    }
     pl->partial_cap = (size_t)std::max<long long>({(long long)rc.nblocks, (long long)rc32.nblocks, (long long)kScratchParts,
-                                                       2LL * 36 * 1024, (long long)pl->n0 * pl->n1});
+                                                       2LL * 36 * 1024, (long long)pl->n0 * pl->n1, (long long)pl->rt[0].nblk,
+                                                       (long long)pl->rt[1].nblk});
   }
   if (hipStreamCreateWithFlags(&pl->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&pl->ev0) != hipSuccess || hipEventCreate(&pl->ev1) != hipSuccess)
@@ -1495,9 +1869,11 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
   HIPCHK(hipMemcpyAsync(pl->st, &s, sizeof(s), hipMemcpyHostToDevice, pl->stream));
   HIPCHK(hipEventRecord(pl->ev0, pl->stream));
   const int per_check = 8;
-  bool x0_zero = false;
-  RETCHK(field_is_zero(pl, x, &x0_zero));
-  if (mode == FH_SOLVE_FP64) {
+  bool x0_zero = false, fused64 = false;
+  RETCHK(solve_start(pl, mode, b, x, &x0_zero, &fused64));
+  if (fused64) {
+    RETCHK(cg_fused64(pl, b, x, x0_zero, s));
+  } else if (mode == FH_SOLVE_FP64) {
     const long long nvp = (nv + 63) / 64 * 64;  // 512-byte aligned sub-buffers
     RETCHK(ensure_work(pl, 3 * (size_t)nvp * sizeof(double)));
     double* r = (double*)pl->work;
@@ -1573,9 +1949,12 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
     HIPCHK(hipMemcpyAsync(p, r, (size_t)nv * sizeof(float), hipMemcpyDeviceToDevice, pl->stream));
     // fused iterations where the fixed-length kernels cover the plan (isotropic coefficient)
     bool fused = pl->fused_cg && pl->op_scale == 1.0;  // the fused step assumes an unscaled G
-    pl->cg_defer = fused && defer_applies(pl);
+    pl->cg_defer = fused && defer_applies<float>(pl);
     pl->defer_nb2 = 0;
     const int gb = grid_blocks(nv);
+    // coupled coefficients read every component's old direction: two direction buffers in turn
+    const bool two = rt_on<float>(pl) && pl->coef_kind != fh::COEF_ISO;
+    const FusedVecs<float> fv{xc, r, {p, two ? Ap : p}, pl->coef32};
     // The single-precision correction c is folded as x += G c, c projected in fp64 (in Ax, free
     // until the true residual overwrites it): rounding in the fp32 recurrence leaves c outside the
     // range of G by about 1e-5 of its size. Folded as it is, that part would enter every later
@@ -1586,7 +1965,8 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
     // direction (p = r).
     auto fold = [&]() -> int {
       if (fused)
-        hipLaunchKernelGGL(fh::k_fold_pending, dim3(gb), dim3(256), 0, pl->stream, nv, Ax, xc, p, pl->st, true);
+        hipLaunchKernelGGL(fh::k_fold_pending, dim3(gb), dim3(256), 0, pl->stream, nv, Ax, xc, fv.p[s.kit & 1], pl->st,
+                           true);
       else
         hipLaunchKernelGGL(fh::k_fold_correction, dim3(gb), dim3(256), 0, pl->stream, nv, Ax, xc, true);
       HIPCHK(hipGetLastError());
@@ -1597,8 +1977,7 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
       return enqueue_true_residual<float>(pl, b, x, Ax, r, false, true);
     };
     // After the first batch (which establishes that the fused kernels cover the plan), a batch of
-    // fused iterations is captured once as a HIP graph (kernel nodes only) and replayed: one
-    // launch per batch instead of seven per iteration. The graph is rebuilt when a buffer moves.
+    // fused iterations is captured once as a HIP graph and replayed (fused_batch)
     int batch = 0;
     pl->last_graph_batches = 0;
     BatchPredictor pred;
@@ -1610,54 +1989,12 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
       len = pred.next(s, std::max(s.tol, s.delta * rmax), per_check);
     };
     for (;; ++batch) {
-      const void* key[5] = {xc, r, p, pl->coef32, pl->spec};
-      if (fused && batch > 0 && pl->use_graphs && !pl->it_graph_off) {
-        if (std::memcmp(key, pl->it_key, sizeof(key)) != 0) drop_graphs(pl);
-        hipGraphExec_t& ex = pl->it_exec[len];
-        if (!ex) {
-          hipGraph_t graph = nullptr;
-          bool all = true;
-          int rc = FH_OK;
-          if (hipStreamBeginCapture(pl->stream, hipStreamCaptureModeRelaxed) != hipSuccess) all = false;
-          for (int k = 0; all && k < len; ++k) {
-            bool ok = false;
-            rc = enqueue_fused_iteration(pl, xc, r, p, pl->coef32, &ok);
-            if (rc != FH_OK || !ok) all = false;
-          }
-          if (all) enqueue_flush(pl);
-          const hipError_t ec = hipStreamEndCapture(pl->stream, &graph);
-          if (all && rc == FH_OK && ec == hipSuccess && graph &&
-              hipGraphInstantiate(&ex, graph, nullptr, nullptr, 0) == hipSuccess) {
-            std::memcpy(pl->it_key, key, sizeof(key));
-          } else {
-            ex = nullptr;
-            pl->it_graph_off = true;  // capture not available here: enqueue the kernels directly
-          }
-          if (graph) (void)hipGraphDestroy(graph);
-          (void)hipGetLastError();
-        }
-        if (ex) {
-          HIPCHK(hipGraphLaunch(ex, pl->stream));
-          ++pl->last_graph_batches;
-          HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
-          HIPCHK(hipStreamSynchronize(pl->stream));
-          if (s.done) break;
-          next_len();
-          if (s.pause) RETCHK(update());
-          continue;
-        }
+      if (fused) {
+        RETCHK(fused_batch<float>(pl, fv, s.kit, len, batch > 0, &fused));
+        if (!fused) pl->cg_defer = false;  // not covered: nothing was enqueued, use the general iteration
       }
-      for (int k = 0; k < len; ++k) {
-        if (fused) {
-          bool ok = false;
-          RETCHK(enqueue_fused_iteration(pl, xc, r, p, pl->coef32, &ok));
-          if (ok) continue;
-          fused = false;  // not covered: nothing was enqueued, use the general iteration
-          pl->cg_defer = false;
-        }
-        RETCHK(enqueue_iteration<float>(pl, xc, r, p, Ap, pl->coef32));
-      }
-      if (fused) enqueue_flush(pl);
+      if (!fused)
+        for (int k = 0; k < len; ++k) RETCHK(enqueue_iteration<float>(pl, xc, r, p, Ap, pl->coef32));
       HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
       HIPCHK(hipStreamSynchronize(pl->stream));
       if (s.done) break;

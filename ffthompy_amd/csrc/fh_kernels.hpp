@@ -676,7 +676,7 @@ static __global__ void k_cg_restart(CGState* st, const double* __restrict__ part
     st->pause = 0;
     st->pend = 0;
     st->bpend = 0;
-    st->xfresh = 1;
+    st->xfresh = st->mixed;  // a correction in single precision starts without a value
     if (st->kit == 0 && hist && st->hist_len > 0) hist[0] = nr;
     st->done = (!(nr > st->tol)) || (st->kit >= st->maxiter);
     st->halt = st->done;
@@ -792,6 +792,14 @@ static __global__ void k_fold_pending(long long n, double* __restrict__ x64, con
   const long long stride = (long long)gridDim.x * blockDim.x;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
     x64[i] = (set ? 0.0 : x64[i]) + (double)((fresh ? 0.0f : x32[i]) + a * p[i]);
+}
+
+// x += alpha p: the pending step of the fused fp64 iteration
+static __global__ void k_fold_step(long long n, double* __restrict__ x, const double* __restrict__ p,
+                                   const CGState* __restrict__ st) {
+  const double a = st->alpha;
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) x[i] += a * p[i];
 }
 
 // x64 += x32 (x64 = x32 with set), x32 = 0 (mixed precision: fold the single-precision correction)

@@ -1,0 +1,106 @@
+// Host side of the runtime-radix passes: radix schedules and launch shapes.
+#include <algorithm>
+
+#include "fh_rt_launch.hpp"
+
+namespace fh {
+namespace rt {
+
+static bool div_exact(long long x, long long d) { return x * d < (1LL << 32); }
+
+// Points per tile (2^lf) of a strided pass of nc components: up to 2^most of nf, fewer until `blocks`
+// workgroups exist (256 CUs, about two workgroups each) and the tile leaves room for other workgroups
+// in LDS. Each butterfly of the longest stage gets a thread where 512 threads allow it.
+static bool pick_cols(const Axis& ax, int nc, size_t rb, long long nf, long long outer, int most, int least,
+                      long long blocks, size_t lds_max, int* lf, int* nthr, int* tpp, size_t* lds) {
+  const int need = threads_need(ax, rb), want = threads_want(ax);
+  for (int l = most; l >= 0; --l) {
+    const long long f = 1LL << l, P = f * nc;
+    *lds = ((size_t)ax.L * P + ax.L) * 2 * rb;
+    const bool fits = P * need <= 512 && *lds <= kLdsUse;
+    const bool small = *lds <= lds_max && ((nf + f - 1) / f * outer >= blocks || l <= least);
+    if (!fits || (!small && l > 0)) continue;
+    *lf = l;
+    *tpp = (int)std::min<long long>(want, 512 / P);
+    *nthr = round64(P * *tpp);
+    return true;
+  }
+  return false;
+}
+
+bool compiled_length(int L) {
+  switch (L) {
+#define FH_RT_CASE(X) case X:
+    FH_RT_LENGTHS(FH_RT_CASE)
+#undef FH_RT_CASE
+    return true;
+    default: return false;
+  }
+}
+
+Config make_config(size_t rb, int n0, int n1, int n2, int nc) {
+  Config c;
+  const bool three = n0 > 1;
+  if (n1 < 2 || n2 < 2 || n2 > 4096 || n1 > 4096 || n0 > 4096) return c;
+  Geo& g = c.g;
+  g.nc = nc;
+  g.n2 = n2;
+  g.n2h = n2 / 2 + 1;
+  g.nrows = (long long)n0 * n1;
+  g.n = g.nrows * n2;
+  g.nh = g.nrows * g.n2h;
+  g.a2 = plan_axis(n2);
+  if (three) g.a1 = plan_axis(n1);
+  c.a0 = plan_axis(three ? n0 : n1);
+  if (!g.a2.nst || !c.a0.nst || (three && !g.a1.nst)) return c;
+  if (!div_exact((long long)n1 * g.n2h, g.n2h)) return c;
+  g.dn2 = make_div(n2);
+  g.dn2h = make_div(g.n2h);
+  if ((unsigned long long)nc * g.nh * 2 * rb >= (1ULL << 31)) return c;  // buffer offsets (see kDead)
+  // Plane mode (the whole plane of one component in LDS) for every compiled plane (135^3: 114 us against
+  // 130 us of row mode in double, 71 against 85 in single precision). A plane of other lengths runs the
+  // schedule-driven kernel: it wins while one round of workgroups covers the chip (63 x 81 x 105, 189
+  // workgroups: 52 against 59 us) and loses beyond (90 x 100 x 77, 270: 70 against 62 us; 105 x 63 x 45
+  // elasticity, 630: 76 against 64 us).
+  g.plane = 0;
+  if (three && div_exact((long long)(n1 + 1) * n2, n2)) set_plane(g, n1, rb, &c.nthr, &c.lds);
+  if (g.plane && !(n1 == n2 && compiled_length(n2)) && n0 * nc > 256) g.plane = 0;
+  if (g.plane) c.nblk = (unsigned)(n0 * nc);
+  if (!g.plane) {
+    // row mode: more rows per workgroup while the chip stays covered
+    int rows = 2;
+    auto blocks = [&](int r) { return (g.nrows + r - 1) / r * nc; };
+    while (2 * rows <= 32 && blocks(2 * rows) >= 1024 && (size_t)(n2 + 2) * (rows | 1) * 2 * rb <= 40 * 1024 &&
+           rows * threads_need(g.a2, rb) <= 512)
+      rows *= 2;
+    set_rows(g, rows);
+    g.tw1_off = 0;
+    c.lds = ((size_t)g.tile + n2) * 2 * rb;
+    const int npr = g.rbe / 2;
+    if (c.lds > kLdsUse || npr * threads_need(g.a2, rb) > 512) return c;
+    g.tpp2 = std::min(threads_want(g.a2), 512 / npr);
+    g.tpp1 = 1;
+    c.nthr = round64(npr * g.tpp2);
+    c.nblk = (unsigned)blocks(rows);
+    if (three && !pick_cols(g.a1, 1, rb, g.n2h, (long long)n0 * nc, rb == 4 ? 5 : 4, rb == 4 ? 3 : 2, 1024, 40 * 1024,
+                            &c.lp1, &c.nthr_1, &c.tpp_1, &c.lds_1))
+      return c;
+  }
+  // Tiles of a strided pass read segments of 64 bytes; 128 where the spectrum exceeds the Infinity Cache
+  // by far (in cache the shorter segments win by 2-6 %: more workgroups, less LDS each).
+  const int seg = (rb == 4 ? 3 : 2) + ((size_t)nc * g.nh * 2 * rb > ((size_t)192 << 20));
+  const long long nf = three ? (long long)n1 * g.n2h : g.n2h;
+  if (!pick_cols(c.a0, nc, rb, nf, 1, seg, 0, 256, 64 * 1024, &c.lf, &c.nthr_g, &c.tpp_g, &c.lds_g)) return c;
+  if (!pick_cols(c.a0, 1, rb, nf, 1, rb == 4 ? 5 : 4, 0, 512, 48 * 1024, &c.lp0, &c.nthr_0, &c.tpp_0, &c.lds_0)) return c;
+  g.dnc = make_div(nc);
+  g.dx = c.nthr % n2;
+  g.drow = c.nthr / n2;
+  g.dk = c.nthr % g.n2h;
+  g.dq = c.nthr / g.n2h;
+  if (!div_exact((long long)c.nblk, nc)) return c;
+  c.ok = true;
+  return c;
+}
+
+}  // namespace rt
+}  // namespace fh

@@ -81,20 +81,26 @@ int fh_plan_ncomp(const fh_plan* plan);
 /* Switch the projection between G1 (primal) and G2 (dual): applications.py:53-56. */
 int fh_plan_set_primaldual(fh_plan* plan, int primaldual);
 /* generic = 1 forces the runtime-radix kernels even where a compile-time specialised
- * schedule exists (lengths 5, 9, 15, 25, 27, 45, 63, 75, 81, 99, 105, 125, 135, 225, 243); used to test
- * one path against the other. No reference counterpart. */
+ * schedule exists (lengths 5, 9, 15, 25, 27, 45, 63, 75, 81, 99, 105, 125, 135, 225, 243) and where the
+ * passes of any smooth length cover the grid; used to test one path against the other. No reference
+ * counterpart. */
 int fh_plan_use_generic(fh_plan* plan, int generic);
 
 /* Iteration variant of the mixed-precision CG (FH_SOLVE_MIXED): fused = 1 (default) runs
  * each single-precision iteration as rows-forward (direction update, pending solution step,
  * a p, partial <p, a p>), strided passes, rows-inverse (r -= alpha G(a p), partial <r, r>),
- * using <p, a p> = <p, G(a p)> for p in the range of G; it applies to isotropic
- * coefficients on the fixed-length kernels and falls back otherwise. fused = 0 keeps the
- * reference's operator-form denominator <p, Afun(p)> (ffthompy/general/solver.py:125-126).
+ * using <p, a p> = <p, G(a p)> for p in the range of G; it covers isotropic and Lame
+ * coefficients on the fixed-length kernels and every kind on the passes of any smooth length, and
+ * falls back otherwise. fused = 0 keeps the reference's operator-form denominator <p, Afun(p)>
+ * (ffthompy/general/solver.py:125-126).
  * fused = 1 (default): on grids of at most 12288 rows (n0 * n1) alpha and beta are formed inside
  * the passes (each forward-pass workgroup sums the inverse pass's partials in one fixed order,
  * block 0 of the first strided pass finalises the state) instead of by two one-workgroup kernels
- * per iteration; fused = 2 keeps those kernels. Plain FP64 solves always use the operator form. */
+ * per iteration (on the passes of any smooth length: wherever a pass has at most 2048 workgroups);
+ * fused = 2 keeps those kernels. Plain FP64 solves (FH_SOLVE_FP64) run the same fused iteration where the
+ * passes of any smooth length serve the plan, b lies in the range of G (checked once per solve, to
+ * 1e-12 of its norm) and neither the residual log nor the iterate callback is set; otherwise, and
+ * with fused = 0, they use the operator form. */
 int fh_plan_set_cg_variant(fh_plan* plan, int fused);
 
 /* Mixed-precision CG with the fused iteration: enable = 1 (default) replays batches of
@@ -337,7 +343,8 @@ int fh_last_solve_updates(const fh_plan* plan, int* n_updates);
  * matvecs on the plan stream, each kernel launched with its own start/stop HIP events
  * (hipExtLaunchKernel: the dispatch's timestamps); returns each pass's average duration in
  * ms and the algorithmic HBM bytes it moves per launch. Needs the fixed-length kernels
- * (FH_ERR_UNSUPPORTED otherwise). y holds the matvec result afterwards. At most max_kernels
+ * (FH_ERR_UNSUPPORTED otherwise), which it times also where the plan's own matvec runs the passes of
+ * any smooth length. y holds the matvec result afterwards. At most max_kernels
  * entries; *nkernels receives the count. No reference counterpart (measurement only). */
 int fh_matvec_profile(fh_plan* plan, int dtype, const void* x, void* y, int nrep, int max_kernels,
                       double* kernel_ms, double* kernel_bytes, int* nkernels);
