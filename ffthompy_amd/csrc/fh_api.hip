@@ -271,10 +271,10 @@ struct fh_plan {
   int band[3] = {0, 0, 0};
   double op_scale = 1.0;         // factor of the operator G A (not of the bare projection)
   // fused mixed CG: a batch of iterations captured once as a HIP graph, replayed per batch
-  // captured batches of 1, 2, 4, 8 fused iterations, by length, precision (0 fp64, 1 fp32) and the
-  // direction buffer that the batch starts from
-  hipGraphExec_t it_exec[9][2][2] = {};
-  const void* it_key[2][5] = {};  // buffers the captured batches were built for, by precision
+  // captured batches of 1, 2, 4, 8 iterations, by length, kind (0 fp64, 1 fp32, 2 and 3 the
+  // same of the potential formulation) and the direction buffer that the batch starts from
+  hipGraphExec_t it_exec[9][4][2] = {};
+  const void* it_key[4][5] = {};  // buffers the captured batches were built for, by kind
   bool it_graph_off = false;     // capture failed on this plan: direct launches from then on
   bool use_graphs = true;        // fh_plan_use_graphs
   int last_graph_batches = 0;    // batches of the last solve replayed from the graph
@@ -661,6 +661,32 @@ int rt_operator_front(fh_plan* pl, const T* x, int kind, const T* coef, const in
   return rt_middle<T>(pl, spec, g, halt);
 }
 
+// Forward transform of A(x) x (kind COEF_NONE: of x) into xhat, every component in one launch per pass.
+template <typename T>
+int rt_forward(fh_plan* pl, int nc, const T* x, const T* coef, int kind, cpx<T>* xhat) {
+  fh::rt::FwdArgs<T> a{};
+  a.in = x;
+  a.coef = coef;
+  a.kind = kind;
+  a.out = xhat;
+  RETCHK(rt_fwd<T>(pl, a, nc, false));
+  if (pl->n0 > 1 && !rt_config<T>(pl).g.plane) RETCHK(rt_cols<T>(pl, 0, 1, nc, xhat, xhat, nullptr, nullptr));
+  return rt_cols<T>(pl, 0, pl->n0 > 1 ? 0 : 1, nc, xhat, xhat, nullptr, nullptr);
+}
+
+// Inverse transform of nc <= ncomp components (times scale); xhat is kept, the plan's spectrum is scratch.
+template <typename T>
+int rt_inverse(fh_plan* pl, int nc, const cpx<T>* xhat, T* x, T scale) {
+  cpx<T>* tmp = reinterpret_cast<cpx<T>*>(pl->spec);
+  RETCHK(rt_cols<T>(pl, 1, pl->n0 > 1 ? 0 : 1, nc, xhat, tmp, nullptr, nullptr));
+  if (pl->n0 > 1 && !rt_config<T>(pl).g.plane) RETCHK(rt_cols<T>(pl, 1, 1, nc, tmp, tmp, nullptr, nullptr));
+  fh::rt::InvArgs<T> a{};
+  a.in = tmp;
+  a.out = x;
+  a.scale = scale;
+  return rt_inv<T>(pl, a, nc, nullptr);
+}
+
 // Inverse pass of the operator from the plan's spectrum, epilogue epi (see k_inv).
 template <typename T>
 int rt_operator_back(fh_plan* pl, T* out, int epi, const T* w, float* r32, fh::CGState* st, const int* halt, int* nb) {
@@ -868,16 +894,7 @@ static int matvec_impl(fh_plan* pl, int dtype, const void* x, void* y, bool with
 
 template <typename T>
 static int rfftn_impl(fh_plan* pl, int ncomp, const T* x, cpx<T>* xhat) {
-  if (rt_on<T>(pl)) {
-    // every component in one launch per pass: the passes' spectrum is the 'r' layout
-    fh::rt::FwdArgs<T> a{};
-    a.in = x;
-    a.kind = fh::COEF_NONE;
-    a.out = xhat;
-    RETCHK(rt_fwd<T>(pl, a, ncomp, false));
-    if (pl->n0 > 1 && !rt_config<T>(pl).g.plane) RETCHK(rt_cols<T>(pl, 0, 1, ncomp, xhat, xhat, nullptr, nullptr));
-    return rt_cols<T>(pl, 0, pl->n0 > 1 ? 0 : 1, ncomp, xhat, xhat, nullptr, nullptr);
-  }
+  if (rt_on<T>(pl)) return rt_forward<T>(pl, ncomp, x, nullptr, fh::COEF_NONE, xhat);  // the 'r' layout itself
   const GParams g = make_gparams(pl, 1.0, 1);
   for (int c = 0; c < ncomp; ++c) {
     cpx<T>* out = xhat + (size_t)c * pl->nh;
@@ -897,17 +914,10 @@ static int irfftn_impl(fh_plan* pl, int ncomp, const cpx<T>* xhat, T* x) {
   const GParams g = make_gparams(pl, 1.0, 1);
   cpx<T>* tmp = reinterpret_cast<cpx<T>*>(pl->spec);
   if (rt_on<T>(pl)) {
-    // as many components at a time as the plan's spectrum holds; the first pass reads xhat
-    for (int c0 = 0; c0 < ncomp; c0 += pl->ncomp) {
-      const int m = std::min(pl->ncomp, ncomp - c0);
-      RETCHK(rt_cols<T>(pl, 1, pl->n0 > 1 ? 0 : 1, m, xhat + (size_t)c0 * pl->nh, tmp, nullptr, nullptr));
-      if (pl->n0 > 1 && !rt_config<T>(pl).g.plane) RETCHK(rt_cols<T>(pl, 1, 1, m, tmp, tmp, nullptr, nullptr));
-      fh::rt::InvArgs<T> a{};
-      a.in = tmp;
-      a.out = x + (size_t)c0 * pl->n;
-      a.scale = T(1.0 / (double)pl->n);
-      RETCHK(rt_inv<T>(pl, a, m, nullptr));
-    }
+    // as many components at a time as the plan's spectrum holds
+    for (int c0 = 0; c0 < ncomp; c0 += pl->ncomp)
+      RETCHK(rt_inverse<T>(pl, std::min(pl->ncomp, ncomp - c0), xhat + (size_t)c0 * pl->nh, x + (size_t)c0 * pl->n,
+                           T(1.0 / (double)pl->n)));
     return FH_OK;
   }
   for (int c = 0; c < ncomp; ++c) {
@@ -957,6 +967,7 @@ static int ensure_hist(fh_plan* pl, int len) {
 // Partials per pass that the deferred alpha/beta of a small grid sums (the forward pass's go to
 // pl->partial[0..kDeferMax), the inverse pass's to pl->partial[kDeferMax..2 kDeferMax)).
 constexpr int kDeferMax = 2048;
+constexpr int kPotDefer = 1024;  // as kDeferMax, in the potential formulation (enqueue_fused_pot)
 
 void drop_graphs(fh_plan* pl);
 
@@ -1099,36 +1110,18 @@ struct FusedVecs {
   const T* coef;
 };
 
-// A batch of `len` fused iterations, the first of them iteration number `kit`, and the flush of a
-// deferred beta. With `graph` the batch is captured once as a HIP graph (kernel nodes only) and
-// replayed: one launch per batch. *ok = false (nothing enqueued) where no fused kernels cover the plan.
-template <typename T>
-static int fused_batch(fh_plan* pl, const FusedVecs<T>& v, int kit, int len, bool graph, bool* ok) {
-  const int prec = sizeof(T) == 8 ? 0 : 1;
-  const int par = v.p[0] == v.p[1] ? 0 : kit & 1;
-  auto enqueue = [&](bool* all) -> int {
-    for (int k = 0; k < len; ++k) {
-      if (rt_on<T>(pl)) {
-        RETCHK(enqueue_fused_rt<T>(pl, v.xc, v.r, v.p[(par + k) & 1], v.p[(par + k + 1) & 1], v.coef));
-        continue;
-      }
-      bool covered = false;
-      if constexpr (sizeof(T) == 4) RETCHK(enqueue_fused_iteration(pl, v.xc, v.r, v.p[0], v.coef, &covered));
-      if (!covered) {
-        *all = false;
-        return FH_OK;
-      }
-    }
-    enqueue_flush(pl);
-    return FH_OK;
-  };
+// A batch of fused iterations (enqueue, which sets its argument false where no fused kernels cover the
+// plan: nothing is enqueued then). With `graph` it is captured once as a HIP graph (kernel nodes only) for
+// the buffers `key` and replayed: one launch per batch.
+template <typename F>
+static int run_batch(fh_plan* pl, int kind, int par, int len, const void* const (&key)[5], bool graph, bool* ok,
+                     const F& enqueue) {
   *ok = true;
-  const void* key[5] = {v.xc, v.r, v.p[0], v.coef, pl->spec};
-  if (std::memcmp(key, pl->it_key[prec], sizeof(key)) != 0) {
+  if (std::memcmp(key, pl->it_key[kind], sizeof(key)) != 0) {
     drop_graphs(pl);
-    std::memcpy(pl->it_key[prec], key, sizeof(key));
+    std::memcpy(pl->it_key[kind], key, sizeof(key));
   }
-  hipGraphExec_t& ex = pl->it_exec[len][prec][par];
+  hipGraphExec_t& ex = pl->it_exec[len][kind][par];
   if ((graph || ex) && pl->use_graphs && !pl->it_graph_off) {
     if (!ex) {
       hipGraph_t gr = nullptr;
@@ -1152,6 +1145,30 @@ static int fused_batch(fh_plan* pl, const FusedVecs<T>& v, int kit, int len, boo
     }
   }
   return enqueue(ok);
+}
+
+// A batch of `len` fused iterations, the first of them iteration number `kit`, and the flush of a
+// deferred beta (see run_batch).
+template <typename T>
+static int fused_batch(fh_plan* pl, const FusedVecs<T>& v, int kit, int len, bool graph, bool* ok) {
+  const int par = v.p[0] == v.p[1] ? 0 : kit & 1;
+  const void* const key[5] = {v.xc, v.r, v.p[0], v.coef, pl->spec};
+  return run_batch(pl, sizeof(T) == 8 ? 0 : 1, par, len, key, graph, ok, [&](bool* all) -> int {
+    for (int k = 0; k < len; ++k) {
+      if (rt_on<T>(pl)) {
+        RETCHK(enqueue_fused_rt<T>(pl, v.xc, v.r, v.p[(par + k) & 1], v.p[(par + k + 1) & 1], v.coef));
+        continue;
+      }
+      bool covered = false;
+      if constexpr (sizeof(T) == 4) RETCHK(enqueue_fused_iteration(pl, v.xc, v.r, v.p[0], v.coef, &covered));
+      if (!covered) {
+        *all = false;
+        return FH_OK;
+      }
+    }
+    enqueue_flush(pl);
+    return FH_OK;
+  });
 }
 
 // One CG iteration in precision T on vectors (x, r, p, Ap); everything halts on st->halt.
@@ -1319,7 +1336,8 @@ int ga_interpolate(fh_ga* ga, const double* x, double* out) {
 
 // ---- potential formulation -----------------------------------------------------------------
 
-fh::pot::PotParams pot_params(const fh_plan* pl) {
+// soa: the gradient spectrum is component-major (the passes of any smooth length).
+fh::pot::PotParams pot_params(const fh_plan* pl, bool soa) {
   fh::pot::PotParams g;
   g.n0 = pl->n0;
   g.n1 = pl->n1;
@@ -1330,12 +1348,149 @@ fh::pot::PotParams pot_params(const fh_plan* pl) {
   g.Y[0] = pl->dim == 3 ? pl->Y[0] : 1.0;
   g.Y[1] = pl->Y[pl->dim == 3 ? 1 : 0];
   g.Y[2] = pl->Y[pl->dim - 1];
+  g.st = soa ? 1 : pl->ncomp;
+  g.sj = soa ? pl->nh : 1;
   g.banded = pl->banded;
   for (int a = 0; a < 3; ++a) {
     g.band[a] = pl->band[a];
     g.tpiY[a] = (double)(2.0L * 3.14159265358979323846264338327950288L / (long double)g.Y[a]);
   }
   return g;
+}
+
+// Arguments of the potential formulation's strided passes of any smooth length that do not depend on
+// the direction.
+fh::rt::PotArgs rt_pot_args(fh_plan* pl, cpx<double>* p, const cpx<double>* r, const int* halt) {
+  const fh::rt::Config& c = rt_config<double>(pl);
+  fh::rt::PotArgs a{};
+  a.data = reinterpret_cast<cpx<double>*>(pl->spec);
+  a.p = p;
+  a.r = r;
+  a.st = pl->st;
+  a.sgn = -1.0;
+  a.partial = pl->partial;
+  a.g = pot_params(pl, true);
+  a.cs = (int)pl->nh;
+  a.es = pl->n0 > 1 ? pl->n1 * pl->n2h : pl->n2h;
+  a.lf = c.lf;
+  a.ntiles = (a.es + (1 << c.lf) - 1) >> c.lf;
+  a.tpp = c.tpp_g;
+  a.dP = fh::rt::make_div((long long)pl->ncomp << c.lf);
+  a.dn2h = c.g.dn2h;
+  a.ax = c.a0;
+  a.tw = twiddles<double>(pl, pl->n0 > 1 ? 0 : 1);
+  a.halt = halt;
+  return a;
+}
+
+int rt_pot_pass(fh_plan* pl, fh::rt::PotArgs& a, int dir) {
+  const fh::rt::Config& c = rt_config<double>(pl);
+  a.dir = dir;
+  return rt_result(fh::rt::launch_pot(pl->ncomp, a, c.nthr_g, c.lds_g, rt_launch(pl)), "potential pass");
+}
+
+// Round trip of the gradient spectrum through a(x) (isotropic coefficient), the strided passes along
+// axis 1 around it where the planes do not fit LDS. partial, bpart, bnp: see TripArgs.
+int rt_pot_trip(fh_plan* pl, const int* halt, double* partial, const double* bpart, int bnp) {
+  const fh::rt::Config& c = rt_config<double>(pl);
+  cpx<double>* spec = reinterpret_cast<cpx<double>*>(pl->spec);
+  const bool axis1 = pl->n0 > 1 && !c.g.plane;
+  if (axis1) RETCHK(rt_cols<double>(pl, 1, 1, pl->ncomp, spec, spec, nullptr, halt));
+  fh::rt::TripArgs t{};
+  t.g = c.g;
+  t.spec = spec;
+  t.coef = plan_coef<double>(pl);
+  t.scale = 1.0 / (double)pl->n;
+  t.partial = partial;
+  t.st = pl->st;
+  t.bpart = bpart;
+  t.bnp = bnp;
+  t.halt = halt;
+  t.tw2 = twiddles<double>(pl, 2);
+  t.tw1 = twiddles<double>(pl, 1);
+  RETCHK(rt_result(fh::rt::launch_trip(c, t, c.nblk, rt_launch(pl)), "round trip pass"));
+  return axis1 ? rt_cols<double>(pl, 0, 1, pl->ncomp, spec, spec, nullptr, halt) : FH_OK;
+}
+
+// The potential operator on the passes of any smooth length: three launches where the planes fit LDS
+// (2-D: rows), two strided passes along axis 1 more otherwise; a coefficient that couples the
+// components goes through the real field.
+int rt_pot_operator(fh_plan* pl, cpx<double>* p, const cpx<double>* r, cpx<double>* out, double* re, const cpx<double>* w, const int* halt,
+                    int* nb) {
+  fh::rt::PotArgs a = rt_pot_args(pl, p, r, halt);
+  RETCHK(rt_pot_pass(pl, a, +1));
+  if (pl->coef_kind == fh::COEF_ISO) {
+    RETCHK(rt_pot_trip(pl, halt, nullptr, nullptr, 0));
+  } else {
+    const int nc = pl->ncomp;
+    const bool axis1 = pl->n0 > 1 && !rt_config<double>(pl).g.plane;
+    cpx<double>* spec = a.data;
+    if (axis1) RETCHK(rt_cols<double>(pl, 1, 1, nc, spec, spec, nullptr, halt));
+    fh::rt::InvArgs<double> b{};
+    b.in = spec;
+    b.out = re;
+    b.scale = 1.0 / (double)pl->n;
+    b.halt = halt;
+    RETCHK(rt_inv<double>(pl, b, nc, nullptr));
+    fh::rt::FwdArgs<double> f{};
+    f.in = re;
+    f.coef = plan_coef<double>(pl);
+    f.kind = pl->coef_kind;
+    f.out = spec;
+    f.halt = halt;
+    RETCHK(rt_fwd<double>(pl, f, nc, false));
+    if (axis1) RETCHK(rt_cols<double>(pl, 0, 1, nc, spec, spec, nullptr, halt));
+  }
+  a.out = out;
+  a.w = w;
+  if (nb) *nb = a.ntiles;
+  return rt_pot_pass(pl, a, -1);
+}
+
+// One fused CG iteration of the potential formulation: three launches (planes in LDS or 2-D). <p, A p> is
+// formed as n <e, a e> of the round trip's field e = F^-1 grad P p, so that the divergence pass knows alpha
+// and updates the residual where it forms A p (A p is never stored; x takes alpha p one iteration late,
+// inside the next gradient pass, which reads p anyhow): 19 scalar spectra of traffic against 23 of the
+// operator, update and two dot products. The partials of alpha and beta are summed by their readers up to
+// kPotDefer of them (each a serial read ahead of a workgroup's loads), by one-workgroup kernels beyond.
+int enqueue_fused_pot(fh_plan* pl, cpx<double>* x, cpx<double>* r, cpx<double>* p) {
+  const int* halt = &pl->st->halt;
+  const int n1 = (int)rt_config<double>(pl).nblk;
+  double *part1 = pl->partial, *part2 = pl->partial + pl->partial_cap / 2;
+  fh::rt::PotArgs a = rt_pot_args(pl, p, r, halt);
+  const bool defer1 = n1 <= kPotDefer, defer2 = a.ntiles <= kPotDefer;
+  a.x = x;
+  a.bpart = defer2 ? part2 : nullptr;
+  a.bnp = a.ntiles;
+  RETCHK(rt_pot_pass(pl, a, +1));
+  RETCHK(rt_pot_trip(pl, halt, part1, a.bpart, a.bnp));
+  if (!defer1)
+    hipLaunchKernelGGL(fh::k_cg_alpha, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, part1, n1);
+  a.upd_r = r;
+  a.partial = part2;
+  a.p1 = part1;
+  a.np1 = defer1 ? n1 : 0;
+  a.defer_beta = defer2;
+  RETCHK(rt_pot_pass(pl, a, -1));
+  if (!defer2)
+    hipLaunchKernelGGL(fh::k_cg_beta, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, part2, a.ntiles);
+  HIPCHK(hipGetLastError());
+  return FH_OK;
+}
+
+// `len` of them and the flush of a deferred beta (see run_batch).
+int fused_pot_batch(fh_plan* pl, cpx<double>* x, cpx<double>* r, cpx<double>* p, int len, bool graph) {
+  const void* const key[5] = {x, r, p, plan_coef<double>(pl), pl->spec};
+  bool ok = true;
+  return run_batch(pl, 2, 0, len, key, graph, &ok, [&](bool*) -> int {
+    for (int k = 0; k < len; ++k) RETCHK(enqueue_fused_pot(pl, x, r, p));
+    const int nt = rt_pot_args(pl, p, r, nullptr).ntiles;
+    if (nt <= kPotDefer)
+      hipLaunchKernelGGL(fh::k_cg_flush, dim3(1), dim3(32), 0, pl->stream, pl->st,
+                         pl->partial + pl->partial_cap / 2, nt);
+    HIPCHK(hipGetLastError());
+    return FH_OK;
+  });
 }
 
 // The potential operator out = P (-div) F A F^-1 grad (P p) on the plan's spectra, p first
@@ -1349,7 +1504,7 @@ template <typename T>
 int pot_operator(fh_plan* pl, cpx<T>* p, const cpx<T>* r, cpx<T>* out, T* re, const cpx<T>* w, const int* halt,
                  int* nb) {
   const int nc = pl->ncomp;
-  const fh::pot::PotParams g = pot_params(pl);
+  const fh::pot::PotParams g = pot_params(pl, false);
   cpx<T>* spec = reinterpret_cast<cpx<T>*>(pl->spec);
   const GParams gp = make_gparams(pl, 1.0);
   const int gb = grid_blocks(pl->nh);
@@ -1647,8 +1802,8 @@ int fh_plan_create(int dim, const int* N, const double* Y, int physics, int prim
       if (fixed && (!c.g.plane || slow_plane)) pl->rt[i].ok = false;
     }
     pl->partial_cap = (size_t)std::max<long long>({(long long)rc.nblocks, (long long)rc32.nblocks, (long long)kScratchParts,
-                                                       2LL * 36 * 1024, (long long)pl->n0 * pl->n1, (long long)pl->rt[0].nblk,
-                                                       (long long)pl->rt[1].nblk});
+                                                       2LL * 36 * 1024, (long long)pl->n0 * pl->n1, 2LL * pl->rt[0].nblk,
+                                                       2LL * pl->rt[1].nblk, 2 * (pl->n0 > 1 ? (long long)pl->n1 : 1) * pl->n2h});
   }
   if (hipStreamCreateWithFlags(&pl->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&pl->ev0) != hipSuccess || hipEventCreate(&pl->ev1) != hipSuccess)
@@ -3480,7 +3635,13 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
     return fail(FH_ERR_UNSUPPORTED, "the residual log (fh_plan_set_residual_log) is kept by fh_cg_solve only");
   const bool mixed = mode == FH_SOLVE_MIXED;
   pl->last_graph_batches = 0;
-  const fh::pot::PotParams g = pot_params(pl);
+  // The double-precision solve runs on the passes of any smooth length (fp64 per iteration: 60 x 50 24
+  // against 96 us, 128^3 116 against 480; on lengths with passes of their own 135^3 139 against 174, 81^3 54
+  // against 69, 45 x 45 24 against 33 us). Mixed precision stays on its passes: the fp32 iterations leave
+  // the potential 1e-7 to 1e-6 off inside the residual's tolerance, and that part is their rounding's.
+  const bool rt64 = rt_on<double>(pl) && !mixed;
+  const bool fused = rt64 && pl->coef_kind == fh::COEF_ISO && pl->fused_cg;
+  const fh::pot::PotParams g = pot_params(pl, rt64);
   const long long nh = pl->nh;
   const long long nhp = (nh + 15) / 16 * 16;  // 256-byte aligned sub-buffers
   const int nc = pl->ncomp;
@@ -3514,15 +3675,41 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
   HIPCHK(hipGetLastError());
   cpx<double>* spec = reinterpret_cast<cpx<double>*>(pl->spec);
   const GParams gp = make_gparams(pl, 1.0);
-  RETCHK(launch_rows_fwd<double>(pl, nc, re, pl->coef64, pl->coef_kind, spec, nullptr));
-  RETCHK(launch_cols<double>(pl, 0, 1, nc, spec, gp, nullptr));
-  if (pl->n0 > 1) RETCHK(launch_cols<double>(pl, 0, 0, nc, spec, gp, nullptr));
+  if (rt64) {
+    RETCHK(rt_forward<double>(pl, nc, re, pl->coef64, pl->coef_kind, spec));
+  } else {
+    RETCHK(launch_rows_fwd<double>(pl, nc, re, pl->coef64, pl->coef_kind, spec, nullptr));
+    RETCHK(launch_cols<double>(pl, 0, 1, nc, spec, gp, nullptr));
+    if (pl->n0 > 1) RETCHK(launch_cols<double>(pl, 0, 0, nc, spec, gp, nullptr));
+  }
   hipLaunchKernelGGL((fh::pot::k_pot_div<double>), grid, block, 0, pl->stream, spec, b, g, 1.0, nullptr, nullptr,
                      nullptr);
-  HIPCHK(hipMemsetAsync(x, 0, (size_t)nh * sizeof(cpx<double>), pl->stream));
   const int* halt = &pl->st->halt;
   const int per_check = 8;
-  if (!mixed) {
+  BatchPredictor pred;
+  int len = per_check;
+  if (fused) {
+    // the plan's own iterate (captured batches keep its address) in the place of A p
+    cpx<double>* r = v1;
+    cpx<double>* p = r + nhp;
+    x = p + nhp;
+    HIPCHK(hipMemsetAsync(x, 0, (size_t)nh * sizeof(cpx<double>), pl->stream));
+    hipLaunchKernelGGL((fh::pot::k_pot_residual<double>), grid, block, 0, pl->stream, b, nullptr, r, g, pl->partial);
+    hipLaunchKernelGGL(fh::k_cg_restart, dim3(1), dim3(256), 0, pl->stream, pl->st, pl->partial, gb, pl->hist, false);
+    HIPCHK(hipGetLastError());
+    for (int batch = 0;; ++batch) {
+      RETCHK(fused_pot_batch(pl, x, r, p, len, batch > 0));
+      HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
+      HIPCHK(hipStreamSynchronize(pl->stream));
+      if (s.done) break;
+      len = pred.next(s, s.tol, per_check);
+    }
+    if (s.pend)
+      hipLaunchKernelGGL(fh::k_fold_step, dim3(grid_blocks(2 * nh)), block, 0, pl->stream, 2 * nh, (double*)x,
+                         (const double*)p, pl->st);
+    HIPCHK(hipGetLastError());
+  } else if (!mixed) {
+    HIPCHK(hipMemsetAsync(x, 0, (size_t)nh * sizeof(cpx<double>), pl->stream));
     cpx<double>* r = v1;
     cpx<double>* p = r + nhp;
     cpx<double>* Ap = p + nhp;
@@ -3533,7 +3720,8 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
     auto batch64 = [&]() -> int {
       for (int k = 0; k < per_check; ++k) {
         int nb = 0;
-        RETCHK(pot_operator<double>(pl, p, r, Ap, re, p, halt, &nb));
+        RETCHK(rt64 ? rt_pot_operator(pl, p, r, Ap, re, p, halt, &nb)
+                    : pot_operator<double>(pl, p, r, Ap, re, p, halt, &nb));
         hipLaunchKernelGGL(fh::k_cg_alpha, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, pl->partial, nb);
         hipLaunchKernelGGL((fh::pot::k_pot_update<double>), grid, block, 0, pl->stream, x, r, p, Ap, g, pl->st,
                            pl->partial);
@@ -3557,29 +3745,34 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
     cpx<float>* Ap = p + nhp;
     cpx<float>* xc = Ap + nhp;
     float* re32 = reinterpret_cast<float*>(re);
+    HIPCHK(hipMemsetAsync(x, 0, (size_t)nh * sizeof(cpx<double>), pl->stream));
     HIPCHK(hipMemsetAsync(xc, 0, (size_t)nh * sizeof(cpx<float>), pl->stream));
     hipLaunchKernelGGL((fh::pot::k_pot_residual<float>), grid, block, 0, pl->stream, b, nullptr, r, g, pl->partial);
     hipLaunchKernelGGL(fh::k_cg_restart, dim3(1), dim3(256), 0, pl->stream, pl->st, pl->partial, gb, pl->hist, false);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(p, r, (size_t)nh * sizeof(cpx<float>), hipMemcpyDeviceToDevice, pl->stream));
     const int fb = grid_blocks(2 * nh);
-    auto batch32 = [&]() -> int {
-      for (int k = 0; k < per_check; ++k) {
-        int nb = 0;
-        RETCHK(pot_operator<float>(pl, p, r, Ap, re32, p, halt, &nb));
-        hipLaunchKernelGGL(fh::k_cg_alpha, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, pl->partial, nb);
-        hipLaunchKernelGGL((fh::pot::k_pot_update<float>), grid, block, 0, pl->stream, xc, r, p, Ap, g, pl->st,
-                           pl->partial);
-        hipLaunchKernelGGL(fh::k_cg_beta, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, pl->partial, gb);
-        HIPCHK(hipGetLastError());
-      }
-      return FH_OK;
-    };
-    for (;;) {
-      RETCHK(batch32());
+    // captured once per length and replayed (see run_batch): x is not touched by a batch
+    const void* const key[5] = {xc, r, p, pl->coef32, pl->spec};
+    for (int batch = 0;; ++batch) {
+      bool ok = true;
+      RETCHK(run_batch(pl, 3, 0, len, key, batch > 0, &ok, [&](bool*) -> int {
+        for (int k = 0; k < len; ++k) {
+          int nb = 0;
+          RETCHK(pot_operator<float>(pl, p, r, Ap, re32, p, halt, &nb));
+          hipLaunchKernelGGL(fh::k_cg_alpha, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, pl->partial, nb);
+          hipLaunchKernelGGL((fh::pot::k_pot_update<float>), grid, block, 0, pl->stream, xc, r, p, Ap, g, pl->st,
+                             pl->partial);
+          hipLaunchKernelGGL(fh::k_cg_beta, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, pl->partial, gb);
+          HIPCHK(hipGetLastError());
+        }
+        return FH_OK;
+      }));
       HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
       HIPCHK(hipStreamSynchronize(pl->stream));
       if (s.done) break;
+      const double rmax = s.pause ? std::sqrt(s.rr) : s.rmax;
+      len = pred.next(s, std::max(s.tol, s.delta * rmax), per_check);
       if (s.pause) {
         hipLaunchKernelGGL(fh::k_fold_correction, dim3(fb), block, 0, pl->stream, 2 * nh, (double*)x, (float*)xc, false);
         RETCHK(pot_operator<double>(pl, x, nullptr, Ax, re, nullptr, nullptr, nullptr));
@@ -3592,16 +3785,20 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
     HIPCHK(hipGetLastError());
   }
   // Fu = P x (homogenisation.py:117); e = F^-1 grad Fu
-  cpx<double>* tmp = v1;
-  hipLaunchKernelGGL(fh::pot::k_pot_precond, grid, block, 0, pl->stream, x, tmp, g);
-  HIPCHK(hipMemcpyAsync(x, tmp, (size_t)nh * sizeof(cpx<double>), hipMemcpyDeviceToDevice, pl->stream));
+  cpx<double>* Fu = reinterpret_cast<cpx<double>*>(Fu_);
+  hipLaunchKernelGGL(fh::pot::k_pot_precond, grid, block, 0, pl->stream, x, Fu, g);
+  HIPCHK(hipGetLastError());
   if (X_) {
-    hipLaunchKernelGGL((fh::pot::k_pot_grad<double>), grid, block, 0, pl->stream, x, spec, g, 0, nullptr);
+    hipLaunchKernelGGL((fh::pot::k_pot_grad<double>), grid, block, 0, pl->stream, Fu, spec, g, 0, nullptr);
     HIPCHK(hipGetLastError());
-    if (pl->n0 > 1) RETCHK(launch_cols<double>(pl, 1, 0, nc, spec, gp, nullptr));
-    RETCHK(launch_cols<double>(pl, 1, 1, nc, spec, gp, nullptr));
-    RETCHK(launch_rows_inv<double>(pl, nc, spec, (double*)X_, 1.0 / (double)pl->n, nullptr, nullptr, nullptr,
-                                   nullptr));
+    if (rt64) {
+      RETCHK(rt_inverse<double>(pl, nc, spec, (double*)X_, 1.0 / (double)pl->n));
+    } else {
+      if (pl->n0 > 1) RETCHK(launch_cols<double>(pl, 1, 0, nc, spec, gp, nullptr));
+      RETCHK(launch_cols<double>(pl, 1, 1, nc, spec, gp, nullptr));
+      RETCHK(launch_rows_inv<double>(pl, nc, spec, (double*)X_, 1.0 / (double)pl->n, nullptr, nullptr, nullptr,
+                                     nullptr));
+    }
   }
   HIPCHK(hipEventRecord(pl->ev1, pl->stream));
   HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));

@@ -22,6 +22,7 @@ struct PotParams {
   int ax0;        // view axis of component 0 (3 - dim)
   double Y[3];    // cell size per view axis
   double tpiY[3]; // 2 pi / Y per view axis (the symbol is 2 pi k / Y)
+  long long st, sj;  // entry t of component j of the gradient spectrum sits at t * st + j * sj
   int banded;     // 1: only |k_a| <= band[a] is kept (the coarse grid of a Ga solve)
   int band[3];
 };
@@ -66,8 +67,8 @@ __device__ __forceinline__ double plane_weight(long long t, const PotParams& g) 
   return (i2 == 0 || ((g.n2 & 1) == 0 && 2 * i2 == g.n2)) ? 1.0 : 2.0;
 }
 
-// spec[t][j] = 2 pi i xi_j (P) u[t]: the gradient of the potential in the operator's spectral
-// layout (frequency-major, components adjacent); with_P multiplies by P first.
+// spec[t][j] = 2 pi i xi_j (P) u[t]: the gradient of the potential in the spectral layout of the passes
+// that follow; with_P multiplies by P first.
 template <typename T>
 __global__ void __launch_bounds__(256)
 k_pot_grad(const cpx<T>* __restrict__ u, cpx<T>* __restrict__ spec, PotParams g, int with_P,
@@ -83,7 +84,7 @@ k_pot_grad(const cpx<T>* __restrict__ u, cpx<T>* __restrict__ spec, PotParams g,
     cpx<T> v = u[t];
     if (with_P) v = mk(T(P) * v.x, T(P) * v.y);
     for (int j = 0; j < g.dim; ++j)
-      spec[t * g.dim + j] = in ? mk(-T(q[j]) * v.y, T(q[j]) * v.x) : mk(T(0), T(0));
+      spec[t * g.st + j * g.sj] = in ? mk(-T(q[j]) * v.y, T(q[j]) * v.x) : mk(T(0), T(0));
   }
 }
 
@@ -105,7 +106,7 @@ k_pot_div(const cpx<T>* __restrict__ spec, cpx<T>* __restrict__ out, PotParams g
     if (grad_symbol<T>(k, g, q, P)) {
       T re = T(0), im = T(0);
       for (int j = 0; j < g.dim; ++j) {
-        const cpx<T> s = spec[t * g.dim + j];
+        const cpx<T> s = spec[t * g.st + j * g.sj];
         re += -T(q[j]) * s.y;
         im += T(q[j]) * s.x;
       }
@@ -124,9 +125,9 @@ k_pot_div(const cpx<T>* __restrict__ spec, cpx<T>* __restrict__ out, PotParams g
   }
 }
 
-// out[t] = P u[t] inside the band, 0 outside (Fu = P x after the solve).
+// out[t] = P u[t] inside the band, 0 outside (Fu = P x after the solve; out may be u).
 static __global__ void __launch_bounds__(256)
-k_pot_precond(const cpx<double>* __restrict__ u, cpx<double>* __restrict__ out, PotParams g) {
+k_pot_precond(const cpx<double>* u, cpx<double>* out, PotParams g) {
   const long long nh = (long long)g.n0 * g.n1 * g.n2h;
   for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < nh;
        t += (long long)gridDim.x * blockDim.x) {

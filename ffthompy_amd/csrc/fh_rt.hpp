@@ -351,6 +351,104 @@ __device__ __forceinline__ void load_tw(const V& v, cpx<T>* twl, const cpx<T>* t
     for (int e = tid; e < n1; e += nthr) twl[v.tw1_off + e] = tw1[e];
 }
 
+// Rows of the tile (real pairs) -> half spectrum: R2C along axis 2 and, in plane mode, the forward
+// transform along axis 1, written to `ro` (the rows' run of one component).
+template <typename T, int CL, int PL>
+__device__ __forceinline__ void forward_rows(const View<T, CL, PL>& vw, const Geo& g, __amdgpu_buffer_rsrc_t ro,
+                                             cpx<T>* s, const cpx<T>* twl, int tid, int nthr) {
+  constexpr unsigned CS = sizeof(cpx<T>);
+  const int n2h = vw.n2h, S = vw.S, L = vw.n2, npr = vw.rbe >> 1;
+  {
+    const int t = quot(tid, vw.dpr), q = tid - t * npr;
+    lds_stages<T, -1, CL, 0, 0>(g.a2, twl, t, q, vw.tpp2, t < vw.tpp2, LdsAcc<T>{s, S});
+  }
+  // untangle the paired rows: in place for the transform along axis 1, else straight to HBM
+  {
+    const int dk = g.dk, dq = g.dq;
+    int q = quot(tid, vw.dn2h), k = tid - q * n2h;
+    while (q < npr) {
+      const cpx<T> Z = s[(int)__umul24(k, S) + q];
+      const cpx<T> Zc = conj(s[(int)__umul24(k ? L - k : 0, S) + q]);
+      const cpx<T> d = Z - Zc;
+      const cpx<T> Ya = T(0.5) * (Z + Zc), Yb = mk(T(0.5) * d.y, T(-0.5) * d.x);
+      if constexpr (PL) {
+        s[(int)__umul24(k, S) + q] = Ya;
+        s[(int)__umul24(tangle_slot1(k, L), S) + q] = Yb;
+      } else {
+        // rows past nr lie outside of the resource (the last workgroup may own fewer)
+        const unsigned o = ((unsigned)(2 * q) * n2h + k) * CS;
+        bstore_c<T>(ro, o, Ya);
+        bstore_c<T>(ro, o + (unsigned)n2h * CS, Yb);
+      }
+      k += dk;
+      q += dq;
+      if (k >= n2h) {
+        k -= n2h;
+        ++q;
+      }
+    }
+  }
+  if constexpr (PL) {
+    __syncthreads();
+    const cpx<T>* tw1 = twl + vw.tw1_off;
+    const int t = quot(tid, vw.dn2h), k = tid - t * n2h;
+    const bool on = t < vw.tpp1;
+    const TangleAcc<T> at{s, S, L};
+    lds_stages<T, -1, CL, 0, 1>(g.a1, tw1, t, k, vw.tpp1, on, at);
+    end_stage<T, -1, CL, 1, false, false>(g.a1, tw1, t, k, vw.tpp1, on, at,
+                                          BufAcc<T>{ro, (unsigned)n2h * CS, (unsigned)k * CS});
+  }
+}
+
+// The inverse: half spectrum `ri` (nr rows) -> rows of the tile.
+template <typename T, int CL, int PL>
+__device__ __forceinline__ void inverse_rows(const View<T, CL, PL>& vw, const Geo& g, __amdgpu_buffer_rsrc_t ri,
+                                             cpx<T>* s, const cpx<T>* twl, int tid, int nthr, int nr) {
+  constexpr unsigned CS = sizeof(cpx<T>);
+  const int n2h = vw.n2h, S = vw.S, L = vw.n2, npr = vw.rbe >> 1;
+  if constexpr (PL) {
+    const cpx<T>* tw1 = twl + vw.tw1_off;
+    const int t = quot(tid, vw.dn2h), k = tid - t * n2h;
+    const bool on = t < vw.tpp1;
+    const TangleAcc<T> at{s, S, L};
+    end_stage<T, +1, CL, 0, false, true>(g.a1, tw1, t, k, vw.tpp1, on,
+                                         BufAcc<T>{ri, (unsigned)n2h * CS, (unsigned)k * CS}, at);
+    lds_stages<T, +1, CL, 1, 0>(g.a1, tw1, t, k, vw.tpp1, on, at);
+  }
+  // Hermitian completion into pencils of two real rows; a row past the end is zero
+  {
+    const int dk = g.dk, dq = g.dq;
+    int q = quot(tid, vw.dn2h), k = tid - q * n2h;
+    while (q < npr) {
+      cpx<T> Ya, Yb;
+      if constexpr (PL) {
+        Ya = s[(int)__umul24(k, S) + q];
+        Yb = s[(int)__umul24(tangle_slot1(k, L), S) + q];
+        if (2 * q + 1 >= nr) Yb = mk(T(0), T(0));
+      } else {
+        const unsigned o = ((unsigned)(2 * q) * n2h + k) * CS;
+        Ya = bload_c<T>(ri, o);
+        Yb = bload_c<T>(ri, o + (unsigned)n2h * CS);
+      }
+      if (k == 0 || 2 * k == L) {
+        s[(int)__umul24(k, S) + q] = mk(Ya.x, Yb.x);
+      } else {
+        s[(int)__umul24(k, S) + q] = mk(Ya.x - Yb.y, Ya.y + Yb.x);
+        s[(int)__umul24(L - k, S) + q] = mk(Ya.x + Yb.y, Yb.x - Ya.y);
+      }
+      k += dk;
+      q += dq;
+      if (k >= n2h) {
+        k -= n2h;
+        ++q;
+      }
+    }
+  }
+  __syncthreads();
+  const int t = quot(tid, vw.dpr), q = tid - t * npr;
+  lds_stages<T, +1, CL, 0, 0>(g.a2, twl, t, q, vw.tpp2, t < vw.tpp2, LdsAcc<T>{s, S});
+}
+
 // ---- forward: A(x) v, R2C along axis 2 (and axis 1) -------------------------------------------
 // UPD 0: v = in. UPD 2 (fused CG): first xc += alpha p_old when a step is pending (xc = alpha p_old
 // while it holds no value), p = r + beta p_old written to pout, v = p, partial sums of <p, A p>.
@@ -372,7 +470,7 @@ __global__ void __launch_bounds__(NT) k_fwd(FwdArgs<T> A) {
   const int rblk = quot(lin, g.dnc), c = lin - rblk * g.nc;  // a plane's components follow each other
   const long long row0 = (long long)rblk * g.rb;
   const int nr = (int)min((long long)g.rb, g.nrows - row0);
-  const int n2 = vw.n2, n2h = vw.n2h, S = vw.S, L = n2, npr = vw.rbe >> 1;
+  const int n2 = vw.n2, n2h = vw.n2h, S = vw.S;
   const long long v0 = row0 * n2, n = g.n;
   T bta = T(0), alp = T(0);
   bool fold = false, fresh = false;
@@ -488,48 +586,8 @@ __global__ void __launch_bounds__(NT) k_fwd(FwdArgs<T> A) {
     }
   }
   __syncthreads();
-  {
-    const int t = quot(tid, vw.dpr), q = tid - t * npr;
-    lds_stages<T, -1, CL, 0, 0>(g.a2, twl, t, q, vw.tpp2, t < vw.tpp2, LdsAcc<T>{s, S});
-  }
-  // untangle the paired rows: in place for the transform along axis 1, else straight to HBM
-  const __amdgpu_buffer_rsrc_t ro =
-      make_rsrc(A.out + (long long)c * g.nh + row0 * n2h, (unsigned long long)nr * n2h * CS);
-  {
-    const int dk = g.dk, dq = g.dq;
-    int q = quot(tid, vw.dn2h), k = tid - q * n2h;
-    while (q < npr) {
-      const cpx<T> Z = s[(int)__umul24(k, S) + q];
-      const cpx<T> Zc = conj(s[(int)__umul24(k ? L - k : 0, S) + q]);
-      const cpx<T> d = Z - Zc;
-      const cpx<T> Ya = T(0.5) * (Z + Zc), Yb = mk(T(0.5) * d.y, T(-0.5) * d.x);
-      if constexpr (PL) {
-        s[(int)__umul24(k, S) + q] = Ya;
-        s[(int)__umul24(tangle_slot1(k, L), S) + q] = Yb;
-      } else {
-        // rows past nr lie outside of the resource (the last workgroup may own fewer)
-        const unsigned o = ((unsigned)(2 * q) * n2h + k) * CS;
-        bstore_c<T>(ro, o, Ya);
-        bstore_c<T>(ro, o + (unsigned)n2h * CS, Yb);
-      }
-      k += dk;
-      q += dq;
-      if (k >= n2h) {
-        k -= n2h;
-        ++q;
-      }
-    }
-  }
-  if constexpr (PL) {
-    __syncthreads();
-    const cpx<T>* tw1 = twl + vw.tw1_off;
-    const int t = quot(tid, vw.dn2h), k = tid - t * n2h;
-    const bool on = t < vw.tpp1;
-    const TangleAcc<T> at{s, S, L};
-    lds_stages<T, -1, CL, 0, 1>(g.a1, tw1, t, k, vw.tpp1, on, at);
-    end_stage<T, -1, CL, 1, false, false>(g.a1, tw1, t, k, vw.tpp1, on, at,
-                                   BufAcc<T>{ro, (unsigned)n2h * CS, (unsigned)k * CS});
-  }
+  forward_rows<T, CL, PL>(vw, g, make_rsrc(A.out + (long long)c * g.nh + row0 * n2h, (unsigned long long)nr * n2h * CS),
+                          s, twl, tid, nthr);
   if constexpr (UPD == 2) {
     const double bs = block_sum(acc);
     if (tid == 0) A.partial[blockIdx.x] = bs;
@@ -554,53 +612,11 @@ __global__ void __launch_bounds__(NT) k_inv(InvArgs<T> A) {
   const int rblk = quot(lin, g.dnc), c = lin - rblk * g.nc;
   const long long row0 = (long long)rblk * g.rb;
   const int nr = (int)min((long long)g.rb, g.nrows - row0);
-  const int n2 = vw.n2, n2h = vw.n2h, S = vw.S, L = n2, npr = vw.rbe >> 1;
+  const int n2 = vw.n2, n2h = vw.n2h, S = vw.S;
   load_tw<T>(vw, twl, A.tw2, A.tw1, g.a1.L, tid, nthr);
   const __amdgpu_buffer_rsrc_t ri =
       make_rsrc(A.in + (long long)c * g.nh + row0 * n2h, (unsigned long long)nr * n2h * CS);
-  if constexpr (PL) {
-    const cpx<T>* tw1 = twl + vw.tw1_off;
-    const int t = quot(tid, vw.dn2h), k = tid - t * n2h;
-    const bool on = t < vw.tpp1;
-    const TangleAcc<T> at{s, S, L};
-    end_stage<T, +1, CL, 0, false, true>(g.a1, tw1, t, k, vw.tpp1, on,
-                                  BufAcc<T>{ri, (unsigned)n2h * CS, (unsigned)k * CS}, at);
-    lds_stages<T, +1, CL, 1, 0>(g.a1, tw1, t, k, vw.tpp1, on, at);
-  }
-  // Hermitian completion into pencils of two real rows; a row past the end is zero
-  {
-    const int dk = g.dk, dq = g.dq;
-    int q = quot(tid, vw.dn2h), k = tid - q * n2h;
-    while (q < npr) {
-      cpx<T> Ya, Yb;
-      if constexpr (PL) {
-        Ya = s[(int)__umul24(k, S) + q];
-        Yb = s[(int)__umul24(tangle_slot1(k, L), S) + q];
-        if (2 * q + 1 >= nr) Yb = mk(T(0), T(0));
-      } else {
-        const unsigned o = ((unsigned)(2 * q) * n2h + k) * CS;
-        Ya = bload_c<T>(ri, o);
-        Yb = bload_c<T>(ri, o + (unsigned)n2h * CS);
-      }
-      if (k == 0 || 2 * k == L) {
-        s[(int)__umul24(k, S) + q] = mk(Ya.x, Yb.x);
-      } else {
-        s[(int)__umul24(k, S) + q] = mk(Ya.x - Yb.y, Ya.y + Yb.x);
-        s[(int)__umul24(L - k, S) + q] = mk(Ya.x + Yb.y, Yb.x - Ya.y);
-      }
-      k += dk;
-      q += dq;
-      if (k >= n2h) {
-        k -= n2h;
-        ++q;
-      }
-    }
-  }
-  __syncthreads();
-  {
-    const int t = quot(tid, vw.dpr), q = tid - t * npr;
-    lds_stages<T, +1, CL, 0, 0>(g.a2, twl, t, q, vw.tpp2, t < vw.tpp2, LdsAcc<T>{s, S});
-  }
+  inverse_rows<T, CL, PL>(vw, g, ri, s, twl, tid, nthr, nr);
   const T scale = A.scale;
   const T alp = A.epi == 2 ? T(A.st->alpha) : T(0);
   const long long o0 = (long long)c * g.n + row0 * n2;

@@ -1,4 +1,4 @@
-// Launchers of the runtime-radix passes for one precision (included by fh_rt_f32.hip, fh_rt_f64.hip).
+// Launchers of the runtime-radix passes for one precision (included by the translation units of each pass).
 #pragma once
 #include <hip/hip_ext.h>
 
@@ -81,7 +81,7 @@ hipError_t launch_inv(const Config& c, const InvArgs<T>& a, unsigned nblk, const
     default: return inv_go<T, 0>(c, x, nblk, s);
   }
 }
-#undef FH_RT_GO
+
 
 template <typename T, int CL>
 hipError_t cols_go(int nc, int mode, ColArgs<T>& x, unsigned nblk, int nthr, size_t lds, const Launch& s) {

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "fh_kernels.hpp"
+#include "fh_pot.hpp"
 
 namespace fh {
 namespace rt {
@@ -253,6 +254,50 @@ struct Config {
   size_t lds_0 = 0;
 };
 
+// Potential formulation: the strided pass along the outermost axis fused with the scalar <-> gradient
+// spectra. dir +1: p = r + beta p (r set), gradient of P p, inverse transform into data; dir -1: forward
+// transform of data, o = sgn P div. The operator form stores o in out and sums the weighted <o, w>.
+// A CG iteration (x set / upd_r set) adds the pending alpha p to x in dir +1 and takes r -= alpha o with
+// the weighted <r, r> in dir -1, where every workgroup forms alpha from the round trip's np1 partials p1
+// (0: it is final in *st) and block 0 finalises it; bpart/bnp: the deferred beta, as in FwdArgs.
+struct PotArgs {
+  int dir;
+  cpx<double>* data;
+  cpx<double>* p;
+  const cpx<double>* r;
+  cpx<double>* x;
+  CGState* st;
+  double sgn;
+  cpx<double>* out;
+  const cpx<double>* w;
+  cpx<double>* upd_r;
+  double* partial;
+  const double *p1, *bpart;
+  int np1, bnp, defer_beta;
+  pot::PotParams g;
+  int cs, es, lf, ntiles, tpp;  // component and axis stride (points), log2 of the tile's points
+  Div dP, dn2h;
+  Axis ax;
+  const cpx<double>* tw;
+  const int* halt;
+};
+
+// Round trip in place on a component-major spectrum: C2R (axis 1 too in plane mode) times scale, times
+// a(x), and back. With partial set it also sums n <e, a e> of its field e; block 0 finalises a
+// deferred beta.
+struct TripArgs {
+  Geo g;
+  cpx<double>* spec;
+  const double* coef;
+  double scale;
+  double* partial;
+  CGState* st;
+  const double* bpart;
+  int bnp;
+  const int* halt;
+  const cpx<double>*tw2, *tw1;
+};
+
 // Whether length L is in FH_RT_LENGTHS.
 bool compiled_length(int L);
 
@@ -275,6 +320,9 @@ hipError_t launch_inv(const Config& c, const InvArgs<T>& a, unsigned nblk, const
 // components); mode 2: the projection.
 template <typename T>
 hipError_t launch_cols(int nc, int mode, const ColArgs<T>& a, unsigned nblk, int nthr, size_t lds, const Launch& s);
+
+hipError_t launch_pot(int nc, const PotArgs& a, int nthr, size_t lds, const Launch& s);
+hipError_t launch_trip(const Config& c, const TripArgs& a, unsigned nblk, const Launch& s);
 
 #define FH_RT_EXTERN(T)                                                                                           \
   extern template hipError_t launch_fwd<T>(const Config&, const FwdArgs<T>&, bool, unsigned, const Launch&);     \
