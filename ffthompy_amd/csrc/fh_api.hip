@@ -1287,6 +1287,7 @@ int quadrature_length(int N) {
 // Inverse real FFT of one spectrum component held in `spec` (the plan's half-spectrum layout,
 // transformed in place) to `out`, scaled by `scale`.
 int spec_to_real(fh_plan* pl, cpx<double>* spec, double* out, double scale) {
+  if (rt_on<double>(pl)) return rt_inverse<double>(pl, 1, spec, out, scale);
   const GParams g = make_gparams(pl, 1.0, 1);
   if (pl->n0 > 1) {
     RETCHK(launch_cols<double>(pl, 1, 0, 1, spec, g, nullptr));
@@ -1315,12 +1316,106 @@ int ga_alloc_coef(fh_ga* ga, int kind, int ncoef) {
   return FH_OK;
 }
 
+// Interpolation of a coarse field up to the last axis on the padded passes: the field's spectra as
+// (ncomp, m0, m1, n2/2+1) into y; *ok = false (nothing enqueued) where a pass does not cover the grids.
+// Everything runs on the coarse plan's stream.
+int ga_pad_passes(fh_ga* ga, const double* x, cpx<double>* y, bool* ok) {
+  fh_plan *c = ga->coarse, *f = ga->fine;
+  *ok = false;
+  if (c->generic || f->generic || c->n2 < 2 || c->n1 < 2 || (c->n0 > 1) != (f->n0 > 1)) return FH_OK;
+  const bool three = c->n0 > 1;
+  const int nc = c->ncomp;
+  fh::rt::PadArgs a0{}, a1{};
+  unsigned nb0 = 0, nb1 = 0;
+  int nt0 = 0, nt1 = 0;
+  size_t l0 = 0, l1 = 0;
+  if (three && !fh::rt::pad_config(f->n0, c->n1 * c->n2h, nc, &a0, &nb0, &nt0, &l0)) return FH_OK;
+  if (!fh::rt::pad_config(f->n1, c->n2h, (long long)nc * f->n0, &a1, &nb1, &nt1, &l1)) return FH_OK;
+  *ok = true;
+  cpx<double>* cs = reinterpret_cast<cpx<double>*>(c->spec);
+  RETCHK(rfftn_impl<double>(c, nc, x, cs));
+  const fh::rt::Launch ln{c->stream, nullptr, nullptr};
+  a1.src = cs;
+  a1.scale = 1.0 / (double)c->n;
+  if (three) {
+    a0.src = cs;
+    a0.dst = reinterpret_cast<cpx<double>*>(f->spec);  // (ncomp, m0, n1, n2/2+1): less than the plan's spectrum
+    a0.n = c->n0;
+    a0.scale = a1.scale;
+    a0.tw = twiddles<double>(f, 0);
+    RETCHK(rt_result(fh::rt::launch_pad(a0, nb0, nt0, l0, ln), "padded pass (axis 0)"));
+    a1.src = a0.dst;
+    a1.scale = 1.0;
+  }
+  a1.dst = y;
+  a1.n = c->n1;
+  a1.tw = twiddles<double>(f, 1);
+  return rt_result(fh::rt::launch_pad(a1, nb1, nt1, l1, ln), "padded pass (axis 1)");
+}
+
+// The last pass over `npencils` components at y: fields to out (STORE) or the energies' partial sums of
+// *nb workgroups to the fine plan's buffer. *ok = false where it does not cover the grid.
+int ga_rows_pass(fh_ga* ga, const cpx<double>* y, double* out, int* nb, bool* ok) {
+  fh_plan *c = ga->coarse, *f = ga->fine;
+  const int nc = c->ncomp;
+  fh::rt::GaRowArgs a{};
+  int nthr = 0;
+  size_t lds = 0;
+  *ok = (out || nc != 6) && (out || ga->coef_kind != fh::COEF_LAME) && f->n2 >= 2 * c->n2h - 1 &&
+        fh::rt::ga_rows_config(f->n2, out ? nc : nc * nc, &a, &nthr, &lds);
+  if (!*ok || !y) return FH_OK;
+  a.src = y;
+  a.nrows = (long long)f->n0 * f->n1;
+  a.cs = a.nrows * c->n2h;
+  a.ngroups = (a.nrows + 1) / 2;
+  a.nvox = f->n;
+  a.n2 = c->n2;
+  a.n2h = c->n2h;
+  a.dn2h = fh::rt::make_div(c->n2h);
+  a.kind = ga->coef_kind;
+  a.tw = twiddles<double>(f, 2);
+  a.coef = ga->coef;
+  a.partial = f->partial;
+  a.out = out;
+  // energies: one round of persistent workgroups (what LDS and 2048 threads let 256 CUs hold), each with one
+  // partial sum per entry
+  const long long held = std::max<long long>(1, std::min<long long>({4, (long long)(160 * 1024 / (lds + 2048)), 2048 / nthr}));
+  const unsigned grid = (unsigned)std::min<long long>(a.ngroups, out ? 0x7fffffff : 256 * held);
+  if (nb) *nb = (int)grid;
+  return rt_result(fh::rt::launch_ga_rows(nc, out != nullptr, a, grid, nthr, lds,
+                                          fh::rt::Launch{c->stream, nullptr, nullptr}), "interpolated rows");
+}
+
+int ga_fields(fh_ga* ga, size_t bytes) {
+  if (ga->fields_bytes >= bytes) return FH_OK;
+  if (ga->fields) (void)hipFree(ga->fields);
+  ga->fields = nullptr;
+  ga->fields_bytes = 0;
+  HIPCHK(hipMalloc(&ga->fields, bytes));
+  ga->fields_bytes = bytes;
+  return FH_OK;
+}
+
 // Trigonometric interpolation of one coarse field (ncomp components) onto the quadrature grid.
 int ga_interpolate(fh_ga* ga, const double* x, double* out) {
   fh_plan* c = ga->coarse;
   fh_plan* f = ga->fine;
   cpx<double>* cs = reinterpret_cast<cpx<double>*>(c->spec);
   cpx<double>* fs = reinterpret_cast<cpx<double>*>(f->spec);
+  bool ok = false;
+  RETCHK(ga_rows_pass(ga, nullptr, out, nullptr, &ok));
+  if (ok) {
+    // (ncomp, m0, m1, n2/2+1) fits the fine plan's spectrum beside the first pass's output where both do:
+    // n1 + m1 <= 2 m1 rows of n2h <= m2h / 2 + 1 values
+    const size_t first = (size_t)c->ncomp * f->n0 * c->n1 * c->n2h, all = (size_t)c->ncomp * f->n0 * f->n1 * c->n2h;
+    ok = first + all <= (size_t)f->ncomp * f->nh;
+    if (ok) RETCHK(ga_pad_passes(ga, x, fs + first, &ok));
+    if (ok) {
+      RETCHK(ga_rows_pass(ga, fs + first, out, nullptr, &ok));
+      HIPCHK(hipStreamSynchronize(c->stream));
+      return FH_OK;
+    }
+  }
   const int nb = grid_blocks(f->nh, 256, 8192);
   for (int k = 0; k < c->ncomp; ++k) {
     RETCHK(rfftn_impl<double>(c, 1, x + (size_t)k * c->n, cs));
@@ -3261,15 +3356,29 @@ int fh_ga_energy(fh_ga* ga, const void* const* fields, int nf, double* AH) {
   if (!ga->coef_kind) return fail(FH_ERR_STATE, "Ga coefficient not set");
   for (int i = 0; i < nf; ++i)
     if (!fields[i]) return fail(FH_ERR_ARG, "null field pointer");
-  const size_t per = (size_t)nc * ga->fine->n;
-  const size_t bytes = (size_t)nf * per * sizeof(double);
-  if (ga->fields_bytes < bytes) {
-    if (ga->fields) (void)hipFree(ga->fields);
-    ga->fields = nullptr;
-    ga->fields_bytes = 0;
-    HIPCHK(hipMalloc(&ga->fields, bytes));
-    ga->fields_bytes = bytes;
+  fh_plan *c = ga->coarse, *f = ga->fine;
+  bool ok = false;
+  int nb = 0;
+  RETCHK(ga_rows_pass(ga, nullptr, nullptr, nullptr, &ok));
+  if (ok && (size_t)2 * nf * nf * 1024 <= f->partial_cap) {
+    // spectra up to the last axis of every load, then one pass to the energies (half the memory of the
+    // interpolated fields)
+    const size_t per = (size_t)nc * f->n0 * f->n1 * c->n2h;
+    RETCHK(ga_fields(ga, nf * per * sizeof(cpx<double>)));
+    cpx<double>* y = reinterpret_cast<cpx<double>*>(ga->fields);
+    for (int i = 0; i < nf && ok; ++i) RETCHK(ga_pad_passes(ga, (const double*)fields[i], y + i * per, &ok));
+    if (ok) {
+      RETCHK(ga_rows_pass(ga, y, nullptr, &nb, &ok));
+      hipLaunchKernelGGL(fh::k_energy_final, dim3(1), dim3(256), 0, c->stream, f->partial, nb, nf * nf,
+                         1.0 / (double)f->n, f->aux);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipMemcpyAsync(AH, f->aux, nf * nf * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+      HIPCHK(hipStreamSynchronize(c->stream));
+      return FH_OK;
+    }
   }
+  const size_t per = (size_t)nc * f->n;
+  RETCHK(ga_fields(ga, (size_t)nf * per * sizeof(double)));
   std::vector<const void*> ptr(nf);
   for (int i = 0; i < nf; ++i) {
     RETCHK(ga_interpolate(ga, (const double*)fields[i], ga->fields + i * per));

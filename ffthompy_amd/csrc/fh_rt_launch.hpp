@@ -298,6 +298,39 @@ struct TripArgs {
   const cpx<double>*tw2, *tw1;
 };
 
+// Quadrature lengths with compiled-in passes of the Ga energies: about twice the method's odd lengths.
+#define FH_GA_LENGTHS(X) \
+  X(18) X(30) X(42) X(50) X(54) X(66) X(70) X(78) X(90) X(98) X(110) X(126) X(130) X(150) X(162) X(198) X(210) X(234) \
+  X(250) X(270)
+
+// Zero-padded inverse transform along one axis (see k_pad): outer slabs of n x es -> L x es points.
+struct PadArgs {
+  const cpx<double>* src;
+  cpx<double>* dst;
+  int n, es, lf, ntiles, tpp;
+  double scale;
+  Div dtiles;
+  Axis ax;
+  const cpx<double>* tw;
+};
+
+// Last transform of the interpolation (see k_ga_rows): components cs points apart.
+struct GaRowArgs {
+  const cpx<double>* src;
+  long long cs, nrows, ngroups, nvox;
+  int n2, n2h, tpp, kind;
+  Div dn2h;
+  Axis ax;
+  const cpx<double>* tw;
+  const double* coef;
+  double* partial;
+  double* out;
+};
+
+// Launch shapes of the two; false where a pass does not exist for the length.
+bool pad_config(int L, int es, long long outer, PadArgs* a, unsigned* nblk, int* nthr, size_t* lds);
+bool ga_rows_config(int L, int npencils, GaRowArgs* a, int* nthr, size_t* lds);
+
 // Whether length L is in FH_RT_LENGTHS.
 bool compiled_length(int L);
 
@@ -321,6 +354,8 @@ hipError_t launch_inv(const Config& c, const InvArgs<T>& a, unsigned nblk, const
 template <typename T>
 hipError_t launch_cols(int nc, int mode, const ColArgs<T>& a, unsigned nblk, int nthr, size_t lds, const Launch& s);
 
+hipError_t launch_pad(PadArgs a, unsigned nblk, int nthr, size_t lds, const Launch& s);
+hipError_t launch_ga_rows(int nc, bool store, GaRowArgs a, unsigned nblk, int nthr, size_t lds, const Launch& s);
 hipError_t launch_pot(int nc, const PotArgs& a, int nthr, size_t lds, const Launch& s);
 hipError_t launch_trip(const Config& c, const TripArgs& a, unsigned nblk, const Launch& s);
 

@@ -102,5 +102,32 @@ Config make_config(size_t rb, int n0, int n1, int n2, int nc) {
   return c;
 }
 
+bool pad_config(int L, int es, long long outer, PadArgs* a, unsigned* nblk, int* nthr, size_t* lds) {
+  a->ax = plan_axis(L);
+  a->es = es;
+  if (!a->ax.nst || (unsigned long long)L * es * 16 >= (1ULL << 31)) return false;
+  if (!pick_cols(a->ax, 1, 8, es, outer, 3, 2, 1024, 48 * 1024, &a->lf, nthr, &a->tpp, lds)) return false;
+  a->ntiles = (es + (1 << a->lf) - 1) >> a->lf;
+  a->dtiles = make_div(a->ntiles);
+  const long long nb = outer * a->ntiles;
+  if (nb > 0x7fffffffLL || !div_exact(nb, a->ntiles)) return false;
+  *nblk = (unsigned)nb;
+  return true;
+}
+
+bool ga_rows_config(int L, int npencils, GaRowArgs* a, int* nthr, size_t* lds) {
+  a->ax = plan_axis(L);
+  const int need = npencils * threads_need(a->ax, 8);
+  if (!a->ax.nst || need > 512) return false;
+  // About a thread per point of a row (the energies' loop), in whole rounds of the four SIMDs: of
+  // workgroups of five waves at 160 registers a CU held one at a time (270 points: 755 us against 490 us
+  // of four waves).
+  *nthr = round64(std::max(need, std::min(L, 256)));
+  if (*nthr > 256) *nthr = 512;
+  a->tpp = std::min(threads_want(a->ax), *nthr / npencils);
+  *lds = ((size_t)L * (npencils | 1) + L) * 16;
+  return *lds <= kLdsUse;
+}
+
 }  // namespace rt
 }  // namespace fh
