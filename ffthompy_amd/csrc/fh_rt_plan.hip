@@ -22,7 +22,7 @@ static bool pick_cols(const Axis& ax, int nc, size_t rb, long long nf, long long
     if (!fits || (!small && l > 0)) continue;
     *lf = l;
     *tpp = (int)std::min<long long>(want, 512 / P);
-    *nthr = round64(P * *tpp);
+    *nthr = roundw(P * *tpp);
     return true;
   }
   return false;
