@@ -2926,7 +2926,7 @@ int fh_batch_create(int nsamples, const int* dims, const double* Y, fh_batch** o
       t32[id * B::TWS + m] = fh::mk((float)(double)cosl(ang), (float)(double)sinl(ang));
     }
   }
-  const size_t ws64 = (size_t)b->nslots * (6 * nvec + spec64), ws32 = (size_t)b->nslots * 4 * nvec;
+  const size_t ws64 = (size_t)b->nslots * (6 * nvec + spec64), ws32 = (size_t)b->nslots * 3 * nvec;
   hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreate(&b->ev0);
   if (e == hipSuccess) e = hipEventCreate(&b->ev1);
@@ -2966,7 +2966,7 @@ int fh_batch_create(int nsamples, const int* dims, const double* Y, fh_batch** o
   A.ws64 = b->d_ws64;
   A.ws32 = b->d_ws32;
   A.ws64_stride = 6 * nvec + spec64;
-  A.ws32_stride = 4 * nvec;
+  A.ws32_stride = 3 * nvec;
   A.nvec = nvec;
   A.energy = b->d_energy;
   A.kit = b->d_kit;

@@ -13,7 +13,7 @@ namespace {
 struct Slot {
   double *x[2], *b, *r64, *p64, *q64;
   cpx<double>* spec64;
-  float *r32, *p32, *q32, *xc32;
+  float *r32, *p32, *xc32;
 };
 
 __device__ __forceinline__ Slot slot_of(const Args& A) {
@@ -29,8 +29,7 @@ __device__ __forceinline__ Slot slot_of(const Args& A) {
   float* f = A.ws32 + (long long)blockIdx.x * A.ws32_stride;
   s.r32 = f;
   s.p32 = f + A.nvec;
-  s.q32 = f + 2 * A.nvec;
-  s.xc32 = f + 3 * A.nvec;
+  s.xc32 = f + 2 * A.nvec;
   return s;
 }
 
@@ -42,9 +41,11 @@ __device__ __forceinline__ InOp<T> in_op(int mode, int coef, int nv, const T* a)
   o.nv = nv;
   o.e0 = T(0);
   o.e1 = T(0);
-  o.beta = T(0);
+  o.beta = o.alpha = T(0);
+  o.pend = o.fresh = o.first = 0;
   o.v = nullptr;
   o.r = nullptr;
+  o.x = nullptr;
   o.a = a;
   return o;
 }
@@ -54,8 +55,8 @@ __device__ __forceinline__ OutOp<T> out_op(int mode, int nv) {
   OutOp<T> o;
   o.mode = mode;
   o.nv = nv;
+  o.alpha = T(0);
   o.y = nullptr;
-  o.p = nullptr;
   o.b = nullptr;
   o.r32 = nullptr;
   o.r64 = nullptr;
@@ -67,17 +68,18 @@ __device__ __forceinline__ OutOp<T> out_op(int mode, int nv) {
 // two call sites (fp64 or fp32) so that each pass is instantiated once per length.
 enum Phase : int {
   PH_RHS = 0,   // b = G(-c E_L)                        (fp64)
-  PH_ITER,      // q = G(c p), <p, q>                    (fp32 mixed, fp64 plain)
+  PH_ITER,      // x += alpha p, p = r + beta p, r -= alpha' G(c p)   (fp32 mixed, fp64 plain)
   PH_TRUE,      // r = b - G(c x)                        (fp64, mixed only)
   PH_PROJ,      // x = G x                               (fp64, mixed only)
   PH_FOLD,      // d = G d, x += d: the fp32 correction   (fp64, mixed only)
   PH_DONE
 };
 
-// CG state of the load case in progress (uniform over the workgroup)
+// CG state of the load case in progress (uniform over the workgroup). pend: alpha p of the last iteration
+// is not yet in the solution (mixed: in the correction, which holds no value while fresh).
 struct CG {
-  double rr, rr_old, rmax, beta;
-  int kit, nupd, status, first;
+  double rr, rmax, alpha, beta;
+  int kit, nupd, status, first, pend, fresh;
 };
 
 }  // namespace
@@ -133,22 +135,28 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
       cg.nupd = 1;
       cg.status = 0;
       cg.first = 1;
-      cg.beta = 0.0;
-      cg.rr = cg.rr_old = cg.rmax = 0.0;
+      cg.pend = 0;
+      cg.fresh = P.mixed;
+      cg.alpha = cg.beta = 0.0;
+      cg.rr = cg.rmax = 0.0;
       int ph = PH_RHS;
 #pragma unroll 1
       while (ph != PH_DONE) {
         // ---- the matrix-vector product of this phase
-        double acc;
+        double acc, pAp = 0.0;
         if (ph == PH_ITER && P.mixed) {
-          InOp<float> in = in_op<float>(cg.first ? 1 : 2, coef, nv, a32);
+          InOp<float> in = in_op<float>(2, coef, nv, a32);
           in.v = s.p32;
           in.r = s.r32;
+          in.x = s.xc32;
+          in.alpha = (float)cg.alpha;
           in.beta = (float)cg.beta;
+          in.pend = cg.pend;
+          in.fresh = cg.fresh;
+          in.first = cg.first;
           OutOp<float> out = out_op<float>(1, nv);
-          out.y = s.q32;
-          out.p = s.p32;
-          matvec<float, true, VAR>(tk, nullptr, in, out);
+          out.b = out.y = s.r32;
+          matvec<float, true, VAR>(tk, nullptr, in, out, cg.rr, &pAp);
           acc = out.acc;
         } else {
           InOp<double> in = in_op<double>(1, coef, nv, a64);
@@ -159,13 +167,16 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
             in.e1 = L == 1 ? -1.0 : 0.0;
             out.y = s.b;
           } else if (ph == PH_ITER) {
-            in.mode = cg.first ? 1 : 2;
+            in.mode = 2;
             in.v = s.p64;
             in.r = s.r64;
+            in.x = x;
+            in.alpha = cg.alpha;
             in.beta = cg.beta;
+            in.pend = cg.pend;
+            in.first = cg.first;
             out.mode = 1;
-            out.y = s.q64;
-            out.p = s.p64;
+            out.b = out.y = s.r64;
           } else if (ph == PH_TRUE) {
             in.v = x;
             out.mode = 2;
@@ -180,7 +191,7 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
             in.v = x;
             out.y = x;
           }
-          matvec<double, false, VAR>(tk, s.spec64, in, out);
+          matvec<double, false, VAR>(tk, s.spec64, in, out, cg.rr, &pAp);
           acc = out.acc;
         }
         // ---- what follows the product
@@ -191,11 +202,8 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
             x[e] = 0.0;
             if (P.mixed) {
               s.r32[e] = (float)v;
-              s.p32[e] = (float)v;
-              s.xc32[e] = 0.0f;
             } else {
               s.r64[e] = v;
-              s.p64[e] = v;
             }
             a2 += v * v;
           }
@@ -204,38 +212,21 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
           const bool done = !(cg.rmax > P.tol) || P.maxiter <= 0;
           ph = done ? PH_DONE : PH_ITER;
         } else if (ph == PH_ITER) {
-          cg.first = 0;
-          const double pAp = wg_sum(acc) * inv_n;
+          if (cg.pend) cg.fresh = 0;  // the correction was written
+          cg.first = cg.pend = 0;
           if (!(pAp > 0.0) || !isfinite(pAp)) {
             cg.status = 1;
-            if (P.mixed) {
+            if (P.mixed && !cg.fresh) {
               for (int e = tid; e < N; e += NT) x[e] += (double)s.xc32[e];
             }
             ph = P.mixed ? PH_PROJ : PH_DONE;
             continue;
           }
-          const double alpha = cg.rr / pAp;
-          double a2 = 0.0;
-          if (P.mixed) {
-            const float af = (float)alpha;
-            for (int e = tid; e < N; e += NT) {
-              s.xc32[e] += af * s.p32[e];
-              const float r = s.r32[e] - af * s.q32[e];
-              s.r32[e] = r;
-              a2 += (double)r * (double)r;
-            }
-          } else {
-            for (int e = tid; e < N; e += NT) {
-              x[e] += alpha * s.p64[e];
-              const double r = s.r64[e] - alpha * s.q64[e];
-              s.r64[e] = r;
-              a2 += r * r;
-            }
-          }
-          const double rn = wg_sum(a2) * inv_n;
+          cg.alpha = cg.rr / pAp;
+          cg.pend = 1;
+          const double rn = wg_sum(acc) * inv_n;
           cg.kit += 1;
           cg.beta = rn / cg.rr;
-          cg.rr_old = cg.rr;
           cg.rr = rn;
           const double nr = sqrt(rn);
           const bool conv = !(nr > P.tol), maxed = cg.kit >= P.maxiter;
@@ -245,13 +236,16 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
               // precision), is added to x; b - A x follows in fp64. Rounding leaves the correction
               // outside the range of G by about 1e-5 of its size: added unprojected, that part
               // would enter the later true residuals and be offset by an error inside the range
-              for (int e = tid; e < N; e += NT) {
-                s.q64[e] = (double)s.xc32[e];
-                s.xc32[e] = 0.0f;
-              }
+              const float af = (float)cg.alpha;
+#pragma unroll 4
+              for (int e = tid; e < N; e += NT) s.q64[e] = (double)((cg.fresh ? 0.0f : s.xc32[e]) + af * s.p32[e]);
+              cg.pend = 0;
+              cg.fresh = 1;
               ph = PH_FOLD;
             }
           } else if (conv || maxed) {
+#pragma unroll 4
+            for (int e = tid; e < N; e += NT) x[e] += cg.alpha * s.p64[e];
             ph = PH_DONE;
           }
         } else if (ph == PH_FOLD) {
@@ -263,6 +257,7 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
           // removed a part of the correction): the search direction restarts from it (p = r)
           const double rt = wg_sum(acc) * inv_n;
           cg.beta = 0.0;
+          cg.first = 1;
           cg.rr = rt;
           cg.rmax = sqrt(rt);
           cg.nupd += 1;

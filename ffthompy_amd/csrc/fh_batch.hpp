@@ -18,6 +18,10 @@
 //              first inverse stage, inverse transform.
 //   rows_inv : per row, Z = U + i V rebuilt with Hermitian symmetry, inverse transform;
 //              real and imaginary parts are the two output components.
+// The CG iteration needs two of these passes only: the direction and the solution (one step late) are updated
+// where rows_fwd reads the direction, <p, A p> is taken there, and rows_inv updates the residual in place of
+// storing the product; its traffic is 15 values per voxel against 23 with a sweep of its own for the updates,
+// whose loads and stores of one voxel after another were a chain of trips to memory.
 // The half spectrum (n0 rows of 2*(n1/2+1) complex values, layout [k0][component][k1])
 // sits in LDS in single precision (at most 135 x 136 complex64 = 146880 bytes) and in a
 // per-workgroup global scratch buffer in double precision.
@@ -161,55 +165,85 @@ __device__ __forceinline__ dd wg_sum_dd(dd v) {
 
 // ---- operands of the matrix-vector product --------------------------------------------------
 // Input at voxel vox (both components), times the coefficient c (none, a, or 1/a):
-//   mode 0: the constant field (e0, e1); mode 1: the vector v; mode 2: v <- r + beta v
-//   (the CG direction update, written back) and then v.
+//   mode 0: the constant field (e0, e1); mode 1: the vector v;
+//   mode 2: the CG iteration: the step alpha v that is still missing is added to x (pend; x = alpha v
+//   while x holds no value, fresh), then v <- r + beta v (v <- r with first), written back, and acc += <v, c v>.
+// get() reads what a batch of voxels needs and put() finishes one of them: every load of a batch is in
+// flight before the first store, which the compiler could not reorder (a trip to memory per voxel).
 template <typename T>
 struct InOp {
   int mode, coef, nv;
-  T e0, e1, beta;
+  T e0, e1, beta, alpha;
+  int pend, fresh, first;
   T* v;
   const T* r;
+  T* x;
   const T* a;
-  __device__ __forceinline__ cpx<T> operator()(int vox) const {
-    T v0, v1;
-    if (mode == 0) {
-      v0 = e0;
-      v1 = e1;
-    } else {
-      v0 = v[vox];
-      v1 = v[nv + vox];
-      if (mode == 2) {
-        v0 = r[vox] + beta * v0;
-        v1 = r[nv + vox] + beta * v1;
-        v[vox] = v0;
-        v[nv + vox] = v1;
+  struct Val {
+    T v0, v1, r0, r1, x0, x1, c;
+  };
+  __device__ __forceinline__ Val get(int vox) const {
+    Val u;
+    u.v0 = e0;
+    u.v1 = e1;
+    if (mode != 0 && !(mode == 2 && first && !pend)) {
+      u.v0 = v[vox];
+      u.v1 = v[nv + vox];
+    }
+    if (mode == 2) {
+      u.r0 = r[vox];
+      u.r1 = r[nv + vox];
+      if (pend && !fresh) {
+        u.x0 = x[vox];
+        u.x1 = x[nv + vox];
       }
     }
-    if (coef) {
-      T c = a[vox];
-      if (coef == 2) c = T(1) / c;
-      v0 *= c;
-      v1 *= c;
+    if (coef) u.c = a[vox];
+    return u;
+  }
+  __device__ __forceinline__ cpx<T> put(int vox, const Val& u, double& acc) const {
+    T v0 = u.v0, v1 = u.v1;
+    if (mode == 2) {
+      if (pend) {
+        x[vox] = (fresh ? T(0) : u.x0) + alpha * v0;
+        x[nv + vox] = (fresh ? T(0) : u.x1) + alpha * v1;
+      }
+      v0 = first ? u.r0 : u.r0 + beta * v0;
+      v1 = first ? u.r1 : u.r1 + beta * v1;
+      v[vox] = v0;
+      v[nv + vox] = v1;
     }
-    return mk(v0, v1);
+    T w0 = v0, w1 = v1;
+    if (coef) {
+      T c = u.c;
+      if (coef == 2) c = T(1) / c;
+      w0 *= c;
+      w1 *= c;
+    }
+    if (mode == 2) acc += (double)v0 * (double)w0 + (double)v1 * (double)w1;
+    return mk(w0, w1);
   }
 };
 
-// Output y at voxel vox:
-//   mode 0: y stored; mode 1: y stored and acc += <p, y>;
-//   mode 2 (T = double): t = b - y stored as the residual (fp32 r32 or fp64 r64), acc += t.t
+// Output y at voxel vox, `pre` what pre() read there before the last stage:
+//   mode 0: y stored;
+//   mode 1: r <- r - alpha y (r the residual, in pre), acc += <r, r>;
+//   mode 2 (T = double): t = b - y (b in pre) stored as the residual (fp32 r32 or fp64 r64), acc += t.t
 template <typename T>
 struct OutOp {
   int mode, nv;
+  T alpha;
   T* y;
-  const T* p;
-  const double* b;
+  const T* b;  // mode 1: r; mode 2: b
   float* r32;
   double* r64;
   double acc;
-  __device__ __forceinline__ void operator()(int vox, T y0, T y1) {
+  __device__ __forceinline__ cpx<T> pre(int vox) const {
+    return mode ? mk(b[vox], b[nv + vox]) : mk(T(0), T(0));
+  }
+  __device__ __forceinline__ void operator()(int vox, T y0, T y1, cpx<T> u) {
     if (mode == 2) {
-      const double t0 = b[vox] - (double)y0, t1 = b[nv + vox] - (double)y1;
+      const double t0 = (double)u.x - (double)y0, t1 = (double)u.y - (double)y1;
       if (r32) {
         r32[vox] = (float)t0;
         r32[nv + vox] = (float)t1;
@@ -219,9 +253,13 @@ struct OutOp {
       }
       acc += t0 * t0 + t1 * t1;
     } else {
+      if (mode == 1) {
+        y0 = u.x - alpha * y0;
+        y1 = u.y - alpha * y1;
+        acc += (double)y0 * (double)y0 + (double)y1 * (double)y1;
+      }
       y[vox] = y0;
       y[nv + vox] = y1;
-      if (mode == 1) acc += (double)p[vox] * (double)y0 + (double)p[nv + vox] * (double)y1;
     }
   }
 };
@@ -261,20 +299,39 @@ __device__ __forceinline__ cpx<T>* spec_ptr(cpx<T>* gspec) {
 
 // ---- pass 1: coefficient multiply, forward transform along axis 1, split -------------------
 template <typename T, class FP, bool LDS>
-__device__ __forceinline__ void rows_fwd(const Task& tk, cpx<T>* gspec, const InOp<T>& in) {
+__device__ __forceinline__ double rows_fwd(const Task& tk, cpx<T>* gspec, const InOp<T>& in) {
   constexpr int L = FP::L, TPP = FP::TPP, H = L / 2 + 1, G = NT / TPP, NST = FP::NST;
   static_assert(NST >= 2, "at least two stages");
   cpx<T>* spec = spec_ptr<T, LDS>(gspec);
   const cpx<T>* twl = lds_tw<T>(1);
   const int tid = opaque_tid(), g = tid / TPP, t = tid - g * TPP;
+  double sum = 0.0;
   for (int base = 0; base < tk.n0; base += G) {
     const int i0 = base + g;
     const bool act = g < G && i0 < tk.n0;
     cpx<T>* slot = spec + (long long)(act ? i0 : 0) * (2 * H);
     {
-      FxStage<T, FP, 0, -1> s0;
+      using S0 = FxStage<T, FP, 0, -1>;
+      S0 s0;
       if (act) {
-        s0.load(t, [&](int j) { return in(i0 * L + j); });
+        // all loads of a butterfly in flight, double precision in halves (registers)
+        constexpr int CH = sizeof(T) == 4 ? S0::R : (S0::R + 1) / 2;
+#pragma unroll
+        for (int m = 0; m < S0::M; ++m) {
+          const int i = t + m * TPP;
+          if (S0::valid(i)) {
+#pragma unroll
+            for (int j0 = 0; j0 < S0::R; j0 += CH) {
+              typename InOp<T>::Val u[CH];
+#pragma unroll
+              for (int j = 0; j < CH; ++j)
+                if (j0 + j < S0::R) u[j] = in.get(i0 * L + i + (j0 + j) * S0::B);
+#pragma unroll
+              for (int j = 0; j < CH; ++j)
+                if (j0 + j < S0::R) s0.v[m][j0 + j] = in.put(i0 * L + i + (j0 + j) * S0::B, u[j], sum);
+            }
+          }
+        }
         s0.compute(t, twl);
         s0.store(t, [&](int j, cpx<T> v) { slot[j] = v; });
       }
@@ -305,6 +362,7 @@ __device__ __forceinline__ void rows_fwd(const Task& tk, cpx<T>* gspec, const In
     }
   }
   __syncthreads();
+  return sum;
 }
 
 // G(xi) of the 2-D scalar problem times 1/(n0 n1): G1 = xi xi^T/|xi|^2 (primal),
@@ -442,10 +500,21 @@ __device__ __forceinline__ void rows_inv(const Task& tk, cpx<T>* gspec, OutOp<T>
     __syncthreads();
     stages_ip<T, FP, +1, 1, NST - 1, 1>(t, act, [&](int j, int) -> cpx<T>& { return slot[j]; }, twl);
     if (act) {
-      FxStage<T, FP, NST - 1, +1> sl;
+      using SL = FxStage<T, FP, NST - 1, +1>;
+      SL sl;
+      cpx<T> u[SL::M][SL::R];  // in flight during the stage (outputs sit at i + j p, p = L / R)
+#pragma unroll
+      for (int m = 0; m < SL::M; ++m)
+#pragma unroll
+        for (int j = 0; j < SL::R; ++j)
+          if (SL::valid(t + m * TPP)) u[m][j] = out.pre(i0 * L + t + m * TPP + j * SL::p);
       sl.load(t, [&](int j) { return slot[j]; });
       sl.compute(t, twl);
-      sl.store(t, [&](int j, cpx<T> v) { out(i0 * L + j, v.x, v.y); });
+#pragma unroll
+      for (int m = 0; m < SL::M; ++m)
+#pragma unroll
+        for (int j = 0; j < SL::R; ++j)
+          if (SL::valid(t + m * TPP)) out(i0 * L + t + m * TPP + j * SL::p, sl.v[m][j].x, sl.v[m][j].y, u[m][j]);
     }
   }
   __syncthreads();
@@ -466,16 +535,20 @@ __device__ __forceinline__ void rows_inv(const Task& tk, cpx<T>* gspec, OutOp<T>
 // sizes, so the host picks one by timing (fh_batch_autotune).
 constexpr int NVAR = 2;
 
+// An iteration (out.mode 1) takes alpha = rr / (the scaled sum of <v, c v>) before the last pass; *pAp is that
+// sum, and a breakdown (not positive or not finite) ends the product there.
 template <typename T, bool LDS, int VAR>
-__device__ __forceinline__ void matvec(const Task& tk, cpx<T>* gspec, const InOp<T>& in, OutOp<T>& out) {
+__device__ __forceinline__ void matvec(const Task& tk, cpx<T>* gspec, const InOp<T>& in, OutOp<T>& out, double rr,
+                                       double* pAp) {
   __syncthreads();  // operands written by other threads of the workgroup are complete
+  double sum = 0.0;
   switch (tk.n1) {
 #define X(LEN, FP, FPR)                                        \
   case LEN:                                                    \
     if constexpr (VAR == 0)                                    \
-      rows_fwd<T, FP, LDS>(tk, gspec, in);                     \
+      sum = rows_fwd<T, FP, LDS>(tk, gspec, in);                     \
     else                                                       \
-      rows_fwd<T, FPR, LDS>(tk, gspec, in);                    \
+      sum = rows_fwd<T, FPR, LDS>(tk, gspec, in);                    \
     break;
     FH_BATCH_LENGTHS(X)
 #undef X
@@ -490,6 +563,11 @@ __device__ __forceinline__ void matvec(const Task& tk, cpx<T>* gspec, const InOp
     break;
     FH_BATCH_LENGTHS(X)
 #undef X
+  }
+  if (out.mode == 1) {
+    *pAp = wg_sum(sum) * tk.scale;
+    if (!(*pAp > 0.0) || !isfinite(*pAp)) return;
+    out.alpha = T(rr / *pAp);
   }
   switch (tk.n1) {
 #define X(LEN, FP, FPR)                                        \
