@@ -287,6 +287,30 @@ __device__ __forceinline__ void stages_ip(int t, bool act, Acc&& acc, const cpx<
   }
 }
 
+// Order of a wave's own LDS and global accesses across its lanes (they execute in order; this only keeps the
+// compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The same for one pencil whose threads sit in one wave.
+template <typename T, class FP, int DIR, int S, int SEND, class Acc>
+__device__ __forceinline__ void stages_wave(int t, bool act, Acc&& acc, const cpx<T>* twl) {
+  if constexpr (S < SEND) {
+    FxStage<T, FP, S, DIR> st;
+    if (act) st.load(t, acc);
+    wave_sync();
+    if (act) {
+      st.compute(t, twl);
+      st.store(t, [&](int j, cpx<T> v) { acc(j) = v; });
+    }
+    wave_sync();
+    stages_wave<T, FP, DIR, S + 1, SEND>(t, act, acc, twl);
+  }
+}
+
 template <typename T, bool LDS>
 __device__ __forceinline__ cpx<T>* spec_ptr(cpx<T>* gspec) {
   if constexpr (LDS) {
@@ -298,17 +322,19 @@ __device__ __forceinline__ cpx<T>* spec_ptr(cpx<T>* gspec) {
 }
 
 // ---- pass 1: coefficient multiply, forward transform along axis 1, split -------------------
+// A row's threads sit in one wave (64 / TPP rows a wave), so the stages need no workgroup barriers and the
+// waves drift apart: one's trips to memory overlap another's butterflies.
 template <typename T, class FP, bool LDS>
 __device__ __forceinline__ double rows_fwd(const Task& tk, cpx<T>* gspec, const InOp<T>& in) {
-  constexpr int L = FP::L, TPP = FP::TPP, H = L / 2 + 1, G = NT / TPP, NST = FP::NST;
+  constexpr int L = FP::L, TPP = FP::TPP, H = L / 2 + 1, RW = 64 / TPP, NST = FP::NST;
   static_assert(NST >= 2, "at least two stages");
   cpx<T>* spec = spec_ptr<T, LDS>(gspec);
   const cpx<T>* twl = lds_tw<T>(1);
-  const int tid = opaque_tid(), g = tid / TPP, t = tid - g * TPP;
+  const int tid = opaque_tid(), lane = tid & 63, g = lane / TPP, t = lane - g * TPP;
   double sum = 0.0;
-  for (int base = 0; base < tk.n0; base += G) {
+  for (int base = (tid >> 6) * RW; base < tk.n0; base += NT / 64 * RW) {
     const int i0 = base + g;
-    const bool act = g < G && i0 < tk.n0;
+    const bool act = g < RW && i0 < tk.n0;
     cpx<T>* slot = spec + (long long)(act ? i0 : 0) * (2 * H);
     {
       using S0 = FxStage<T, FP, 0, -1>;
@@ -336,8 +362,8 @@ __device__ __forceinline__ double rows_fwd(const Task& tk, cpx<T>* gspec, const 
         s0.store(t, [&](int j, cpx<T> v) { slot[j] = v; });
       }
     }
-    __syncthreads();
-    stages_ip<T, FP, -1, 1, NST, 1>(t, act, [&](int j, int) -> cpx<T>& { return slot[j]; }, twl);
+    wave_sync();
+    stages_wave<T, FP, -1, 1, NST>(t, act, [&](int j) -> cpx<T>& { return slot[j]; }, twl);
     constexpr int KM = (H + TPP - 1) / TPP;
     cpx<T> U[KM], V[KM];
 #pragma unroll
@@ -351,7 +377,7 @@ __device__ __forceinline__ double rows_fwd(const Task& tk, cpx<T>* gspec, const 
         V[m] = mk(T(0.5) * d.y, T(-0.5) * d.x);
       }
     }
-    __syncthreads();
+    wave_sync();
 #pragma unroll
     for (int m = 0; m < KM; ++m) {
       const int k = t + m * TPP;
@@ -470,13 +496,13 @@ __device__ __forceinline__ void cols_G(const Task& tk, cpx<T>* gspec) {
 // ---- pass 3: Hermitian rebuild, inverse transform along axis 1, output ---------------------
 template <typename T, class FP, bool LDS>
 __device__ __forceinline__ void rows_inv(const Task& tk, cpx<T>* gspec, OutOp<T>& out) {
-  constexpr int L = FP::L, TPP = FP::TPP, H = L / 2 + 1, G = NT / TPP, NST = FP::NST;
+  constexpr int L = FP::L, TPP = FP::TPP, H = L / 2 + 1, RW = 64 / TPP, NST = FP::NST;
   cpx<T>* spec = spec_ptr<T, LDS>(gspec);
   const cpx<T>* twl = lds_tw<T>(1);
-  const int tid = opaque_tid(), g = tid / TPP, t = tid - g * TPP;
-  for (int base = 0; base < tk.n0; base += G) {
+  const int tid = opaque_tid(), lane = tid & 63, g = lane / TPP, t = lane - g * TPP;
+  for (int base = (tid >> 6) * RW; base < tk.n0; base += NT / 64 * RW) {
     const int i0 = base + g;
-    const bool act = g < G && i0 < tk.n0;
+    const bool act = g < RW && i0 < tk.n0;
     cpx<T>* slot = spec + (long long)(act ? i0 : 0) * (2 * H);
     FxStage<T, FP, 0, +1> s0;
     if (act) {
@@ -492,13 +518,13 @@ __device__ __forceinline__ void rows_inv(const Task& tk, cpx<T>* gspec, OutOp<T>
         return mk(u.x - v.y, u.y + v.x);
       });
     }
-    __syncthreads();
+    wave_sync();
     if (act) {
       s0.compute(t, twl);
       s0.store(t, [&](int j, cpx<T> v) { slot[j] = v; });
     }
-    __syncthreads();
-    stages_ip<T, FP, +1, 1, NST - 1, 1>(t, act, [&](int j, int) -> cpx<T>& { return slot[j]; }, twl);
+    wave_sync();
+    stages_wave<T, FP, +1, 1, NST - 1>(t, act, [&](int j) -> cpx<T>& { return slot[j]; }, twl);
     if (act) {
       using SL = FxStage<T, FP, NST - 1, +1>;
       SL sl;
