@@ -311,6 +311,8 @@ struct fh_batch {
   double* d_normres = nullptr;
   int* d_status = nullptr;
   fh::batch::Params* d_par = nullptr;
+  double* d_xs = nullptr;          // one load per task: solutions, then arrivals and status per load
+  int* d_pair = nullptr;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipGraph_t graph = nullptr;
@@ -2857,7 +2859,7 @@ int fh_batch_destroy(fh_batch* b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
   void* bufs[] = {b->d_smp, b->d_order, b->d_counter, b->d_a64, b->d_a32, b->d_tw64, b->d_tw32, b->d_ws64,
-                  b->d_ws32, b->d_energy, b->d_kit, b->d_nupd, b->d_normres, b->d_status, b->d_par};
+                  b->d_ws32, b->d_energy, b->d_kit, b->d_nupd, b->d_normres, b->d_status, b->d_par, b->d_xs, b->d_pair};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
@@ -2912,6 +2914,20 @@ int fh_batch_create(int nsamples, const int* dims, const double* Y, fh_batch** o
     return (long long)sa.n0 * sa.n1 > (long long)sc.n0 * sc.n1;
   });
   b->order_size = order;
+  const bool split = nsamples <= B::kSplitSamples;
+  if (split) {
+    // the two loads of a task follow each other
+    b->ntasks = 4 * nsamples;
+    for (std::vector<int>* o : {&b->order_sample, &b->order_size}) {
+      std::vector<int> two;
+      for (int code : *o) {
+        two.push_back(2 * code);
+        two.push_back(2 * code + 1);
+      }
+      *o = two;
+    }
+    order = b->order_size;
+  }
   int ncu = 0;
   HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, 0));
   b->nslots = std::max(1, std::min(b->ntasks, ncu));
@@ -2945,6 +2961,8 @@ int fh_batch_create(int nsamples, const int* dims, const double* Y, fh_batch** o
   if (e == hipSuccess) e = hipMalloc(&b->d_normres, (size_t)nsamples * 4 * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&b->d_status, (size_t)nsamples * 2 * sizeof(int));
   if (e == hipSuccess) e = hipMalloc(&b->d_par, sizeof(B::Params));
+  if (e == hipSuccess && split) e = hipMalloc(&b->d_xs, (size_t)nsamples * 4 * nvec * sizeof(double));
+  if (e == hipSuccess && split) e = hipMalloc(&b->d_pair, (size_t)nsamples * 6 * sizeof(int));
   if (e == hipSuccess)
     e = hipMemcpy(b->d_smp, b->smp.data(), nsamples * sizeof(B::Sample), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(b->d_order, order.data(), b->ntasks * sizeof(int), hipMemcpyHostToDevice);
@@ -2958,6 +2976,11 @@ int fh_batch_create(int nsamples, const int* dims, const double* Y, fh_batch** o
   A.smp = b->d_smp;
   A.order = b->d_order;
   A.ntasks = b->ntasks;
+  A.split = split;
+  A.npairs = 2 * nsamples;
+  A.xs = b->d_xs;
+  A.pair = b->d_pair;
+  A.lstat = b->d_pair ? b->d_pair + 2 * nsamples : nullptr;
   A.counter = b->d_counter;
   A.a64 = b->d_a64;
   A.a32 = b->d_a32;

@@ -4,8 +4,9 @@
 namespace fh {
 namespace batch {
 
-__global__ void k_batch_reset(int* counter) {
+__global__ void k_batch_reset(int* counter, int* pair, int n) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *counter = 0;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) pair[i] = 0;
 }
 
 namespace {
@@ -96,7 +97,9 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
     const int task = sh_task;
     __syncthreads();
     if (task >= A.ntasks) break;
-    const int code = A.order[task];
+    const int entry = A.order[task];
+    const int code = A.split ? entry >> 1 : entry;
+    const int L0 = A.split ? entry & 1 : 0, L1 = A.split ? L0 + 1 : 2;
     const int si = code >> 1;
     const Sample sm = A.smp[si];
     Task tk;
@@ -127,9 +130,10 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
     const int nv = tk.nv, N = 2 * nv;
     const double inv_n = tk.scale;
     int status = 0;
+    double* const xs0 = A.split ? A.xs + (long long)(base * 2) * A.nvec : s.x[0];  // load 1: nvec further on
 #pragma unroll 1
-    for (int L = 0; L < 2; ++L) {
-      double* x = L ? s.x[1] : s.x[0];
+    for (int L = L0; L < L1; ++L) {
+      double* x = xs0 + L * A.nvec;
       CG cg;
       cg.kit = 0;
       cg.nupd = 1;
@@ -274,14 +278,28 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
       status |= cg.status;
       __syncthreads();
     }
+    if (A.split) {
+      // the second workgroup to finish sees the first one's solution: every wave releases its stores to
+      // the device before the arrival is counted, and acquires after it
+      if (tid == 0) A.lstat[base * 2 + L0] = status;
+      __threadfence();
+      __syncthreads();
+      if (tid == 0) sh_task = atomicAdd(A.pair + base, 1);
+      __syncthreads();
+      const int arrived = sh_task;
+      __syncthreads();
+      if (arrived == 0) continue;
+      __threadfence();
+      status = A.lstat[base * 2] | A.lstat[base * 2 + 1];
+    }
     // energies <c e_i, e_j>, e_i = E_i + x_i (ffthompy/postprocess.py:53-70)
     dd e00, e01, e11;
     e00.hi = e00.lo = e01.hi = e01.lo = e11.hi = e11.lo = 0.0;
     for (int v = tid; v < nv; v += NT) {
       double c = a64[v];
       if (tk.pd) c = 1.0 / c;
-      const double u0 = s.x[0][v] + 1.0, u1 = s.x[0][nv + v];
-      const double w0 = s.x[1][v], w1 = s.x[1][nv + v] + 1.0;
+      const double u0 = xs0[v] + 1.0, u1 = xs0[nv + v];
+      const double w0 = xs0[A.nvec + v], w1 = xs0[A.nvec + nv + v] + 1.0;
       dd t;
       t.lo = 0.0;
       t.hi = c * (u0 * u0 + u1 * u1);
@@ -317,7 +335,8 @@ hipError_t allow_lds(size_t lds) {
 }
 
 hipError_t enqueue(const Args& A, int nslots, size_t lds, hipStream_t stream, int var) {
-  hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, stream, A.counter);
+  const int n = A.split ? A.npairs : 0;
+  hipLaunchKernelGGL(k_batch_reset, dim3((n + 255) / 256 + 1), dim3(256), 0, stream, A.counter, A.pair, n);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (var == 0)

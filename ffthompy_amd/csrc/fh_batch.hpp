@@ -6,7 +6,8 @@
 // CG to an absolute tolerance on sqrt(<r,r>) (ffthompy/general/solver.py:80-139), and
 // the energy matrix <A e_i, e_j> (ffthompy/postprocess.py:53-70). A workgroup of NT
 // threads owns one task at a time and takes the next from a device counter when done, so
-// uneven grids balance over the chip without host round trips.
+// uneven grids balance over the chip without host round trips. Up to kSplitSamples samples a task is one
+// unit load; the workgroup that finishes a sample's second load forms its energies.
 //
 // Matrix-vector product y = F^-1 G F (c x) inside the workgroup, both components of the
 // field at once:
@@ -42,6 +43,10 @@ constexpr int NT = 512;      // threads per workgroup
 constexpr int MAXL = 135;    // longest supported axis
 constexpr int TWS = 136;     // twiddle table slot (entries)
 constexpr int NLEN = 6;      // supported axis lengths
+// One load per task up to this many samples (their solutions take at most 2.4 GB): 32 samples keep 128
+// instead of 64 CUs busy (22.7 -> 11.6 ms), 512 end more evenly (45.8 -> 43.4 ms); beyond, 16 tasks and
+// more per CU balance as they are.
+constexpr int kSplitSamples = 2048;
 constexpr int kLens[NLEN] = {27, 45, 63, 81, 105, 135};
 
 __host__ __device__ constexpr int len_id(int L) {
@@ -72,6 +77,11 @@ struct Args {
   const Sample* smp;
   const int* order;  // task t -> sample * 2 + pd (pd 0 primal, 1 dual), largest grids first
   int ntasks;
+  int split;         // 1: order holds 2 (sample * 2 + pd) + load, xs the solutions, pair the arrivals
+  int npairs;        // 2 * samples
+  double* xs;        // [sample][pd][load] solutions, stride nvec
+  int* pair;         // [sample][pd] loads finished; cleared with the counter
+  int* lstat;        // [sample][pd][load] status
   int* counter;      // next task; cleared by k_batch_reset before every launch
   const double* a64; // conductivity a(x), concatenated over samples, origin-0 C order
   const float* a32;
@@ -608,7 +618,7 @@ __device__ __forceinline__ void matvec(const Task& tk, cpx<T>* gspec, const InOp
   }
 }
 
-__global__ void k_batch_reset(int* counter);
+__global__ void k_batch_reset(int* counter, int* pair, int n);
 template <int VAR>
 __global__ void __launch_bounds__(NT) k_batch_solve(Args A);
 
