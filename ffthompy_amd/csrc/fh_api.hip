@@ -265,6 +265,8 @@ struct fh_plan {
   bool fused_cg = true;          // mixed CG: fused iteration where available
   bool defer_ok = true;          // fused iteration: alpha/beta inside the passes on small grids
   bool cg_defer = false;         // this solve runs the deferred alpha/beta
+  CGState* st_host = nullptr;    // pinned copy of the CG state (k_cg_publish)
+  int pub_nb2[2] = {0, 0};       // the same of the last iteration enqueued or captured, fp64 and fp32
   int defer_nb2 = 0;             // workgroups of the fused inverse row pass (its partials)
   hipEvent_t prof_t0 = nullptr, prof_t1 = nullptr;  // matvec profile: events of the next launch
   int banded = 0;                // 1: projection restricted to |k_a| <= band[a] (view axes)
@@ -1022,7 +1024,7 @@ static int enqueue_fused_rt(fh_plan* pl, T* xc, T* r, T* pin, T* pout, const T* 
   b.halt = halt;
   RETCHK(rt_inv<T>(pl, b, pl->ncomp, nullptr));
   if (defer) {
-    pl->defer_nb2 = nb;
+    pl->pub_nb2[sizeof(T) == 8 ? 0 : 1] = pl->defer_nb2 = nb;
   } else {
     hipLaunchKernelGGL(fh::k_cg_beta, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, part2, nb);
     HIPCHK(hipGetLastError());
@@ -1033,7 +1035,7 @@ static int enqueue_fused_rt(fh_plan* pl, T* xc, T* r, T* pin, T* pout, const T* 
 // One fused fp32 CG iteration. With pl->cg_defer (small grids) alpha and beta have no kernels of
 // their own: the forward row pass takes the previous beta from the inverse pass's partials, block 0
 // of the first strided pass finalises beta and alpha, and the inverse row pass marks its beta as
-// deferred; k_cg_flush finalises the last beta of a batch.
+// deferred; k_cg_publish finalises the last beta of a batch.
 static int enqueue_fused_iteration(fh_plan* pl, float* xc, float* r, float* p, const float* coef, bool* ok) {
   *ok = false;
   if (pl->generic || (pl->coef_kind != fh::COEF_ISO && pl->coef_kind != fh::COEF_LAME)) return FH_OK;
@@ -1090,18 +1092,26 @@ static int enqueue_fused_iteration(fh_plan* pl, float* xc, float* r, float* p, c
   if (rr == 0) return fail(FH_ERR_STATE, "fused rows inverse unavailable");
   RETCHK(fixed_result(rr, "rows inverse (fused)"));
   if (defer)
-    pl->defer_nb2 = nb2;
+    pl->pub_nb2[1] = pl->defer_nb2 = nb2;
   else
     hipLaunchKernelGGL(fh::k_cg_beta, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, part2, nb2);
   HIPCHK(hipGetLastError());
   return FH_OK;
 }
 
-// End of a batch of fused iterations with deferred beta: finalise it for the host.
-static void enqueue_flush(fh_plan* pl) {
-  if (pl->cg_defer)
-    hipLaunchKernelGGL(fh::k_cg_flush, dim3(1), dim3(32), 0, pl->stream, pl->st, pl->partial + kDeferMax,
-                       pl->defer_nb2);
+// After a batch of iterations: finalise a deferred beta (np partials at part, 0: none) and read the state.
+static int read_state(fh_plan* pl, CGState& s, const double* part, int np) {
+  hipLaunchKernelGGL(fh::k_cg_publish, dim3(1), dim3(64), 0, pl->stream, pl->st, part, np, pl->st_host);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(pl->stream));
+  s = *pl->st_host;
+  return FH_OK;
+}
+
+// The same for a solve on the plan's operator in precision T.
+template <typename T>
+static int read_state(fh_plan* pl, CGState& s) {
+  return read_state(pl, s, pl->partial + kDeferMax, pl->cg_defer ? pl->pub_nb2[sizeof(T) == 8 ? 0 : 1] : 0);
 }
 
 // Vectors of a fused solve: the correction (or, in fp64, the iterate), the residual and the two
@@ -1149,8 +1159,7 @@ static int run_batch(fh_plan* pl, int kind, int par, int len, const void* const 
   return enqueue(ok);
 }
 
-// A batch of `len` fused iterations, the first of them iteration number `kit`, and the flush of a
-// deferred beta (see run_batch).
+// A batch of `len` fused iterations, the first of them iteration number `kit` (see run_batch).
 template <typename T>
 static int fused_batch(fh_plan* pl, const FusedVecs<T>& v, int kit, int len, bool graph, bool* ok) {
   const int par = v.p[0] == v.p[1] ? 0 : kit & 1;
@@ -1168,7 +1177,6 @@ static int fused_batch(fh_plan* pl, const FusedVecs<T>& v, int kit, int len, boo
         return FH_OK;
       }
     }
-    enqueue_flush(pl);
     return FH_OK;
   });
 }
@@ -1575,17 +1583,12 @@ int enqueue_fused_pot(fh_plan* pl, cpx<double>* x, cpx<double>* r, cpx<double>* 
   return FH_OK;
 }
 
-// `len` of them and the flush of a deferred beta (see run_batch).
+// `len` of them (see run_batch).
 int fused_pot_batch(fh_plan* pl, cpx<double>* x, cpx<double>* r, cpx<double>* p, int len, bool graph) {
   const void* const key[5] = {x, r, p, plan_coef<double>(pl), pl->spec};
   bool ok = true;
   return run_batch(pl, 2, 0, len, key, graph, &ok, [&](bool*) -> int {
     for (int k = 0; k < len; ++k) RETCHK(enqueue_fused_pot(pl, x, r, p));
-    const int nt = rt_pot_args(pl, p, r, nullptr).ntiles;
-    if (nt <= kPotDefer)
-      hipLaunchKernelGGL(fh::k_cg_flush, dim3(1), dim3(32), 0, pl->stream, pl->st,
-                         pl->partial + pl->partial_cap / 2, nt);
-    HIPCHK(hipGetLastError());
     return FH_OK;
   });
 }
@@ -1661,32 +1664,39 @@ void drop_graphs(fh_plan* pl) {
       }
 }
 
-// Length of the next batch of CG iterations between two host synchronisations: the iterations
-// that the convergence rate since the last synchronisation predicts until the residual norm falls
-// below `target` (the next stop or reliable-update threshold), plus one, rounded up to a power of
-// two within [1, cap] (so that at most four captured batch graphs exist per plan). An iteration
-// enqueued past the stop returns at once on the halt flag but still dispatches its grids (the
-// waste of a fixed batch of 8 is up to 7 iterations at every stop and reliable update); a batch
-// one short costs one more synchronisation.
+// Number of CG iterations up to the next host synchronisation: what the convergence rate since the last
+// one predicts until the residual norm falls below `target` (the next stop or reliable-update threshold),
+// plus one, between 1 and the iterations done so far (8 to 64: a wrong prediction must not double the
+// work). An iteration enqueued past the stop returns at once on the halt flag but still dispatches its
+// grids (2-3 us each); a synchronisation costs 20 us and more. They are enqueued in batches of 8, 4, 2
+// and 1 (captured graphs, four lengths per kind of iteration): 135 x 135 fp64, 40 iterations: 1130 us
+// with a synchronisation and a copied state every 8 of them, 1050 us so.
 struct BatchPredictor {
   double nr_prev = -1.0;
   int kit_prev = 0;
   double rate = -1.0;
-  int next(const CGState& s, double target, int cap) {
+  int next(const CGState& s, double target) {
+    const int cap = std::min(64, std::max(8, s.kit));
     const double nr = std::sqrt(s.rr);
     if (nr_prev > 0.0 && s.kit > kit_prev && nr > 0.0)
       rate = nr < nr_prev ? std::pow(nr / nr_prev, 1.0 / (double)(s.kit - kit_prev)) : -1.0;
     nr_prev = nr;
     kit_prev = s.kit;
-    if (!(rate > 0.0 && rate < 1.0) || !(target > 0.0) || !(nr > target)) return cap;
+    if (!(rate > 0.0 && rate < 1.0) || !(target > 0.0) || !(nr > target)) return 8;
     const double n = std::log(target / nr) / std::log(rate);
-    if (!(n < (double)cap)) return cap;
-    const int want = (int)std::ceil(n) + 1;
-    int len = 1;
-    while (len < want && len < cap) len *= 2;
-    return std::min(len, cap);
+    return n < (double)cap ? std::min(cap, (int)std::ceil(n) + 1) : cap;
   }
 };
+
+// n iterations as batches batch(len, iterations before it) of 8, 4, 2 and 1.
+template <typename F>
+int run_batches(int n, const F& batch) {
+  for (int done = 0, len = 8; done < n; done += len) {
+    while (len > n - done) len /= 2;
+    RETCHK(batch(len, done));
+  }
+  return FH_OK;
+}
 
 // The fp64 CG on fused iterations: the operations of the reference's CG with the solution update one
 // iteration late (inside the next forward pass) and <p, A p> formed there. s: the host copy of the CG
@@ -1712,11 +1722,12 @@ static int cg_fused64(fh_plan* pl, const double* b, double* x, bool x0_zero, CGS
   pl->last_graph_batches = 0;
   for (int batch = 0;; ++batch) {
     bool ok = true;
-    RETCHK(fused_batch<double>(pl, v, s.kit, len, batch > 0, &ok));
-    HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
-    HIPCHK(hipStreamSynchronize(pl->stream));
+    RETCHK(run_batches(len, [&](int m, int done) {
+      return fused_batch<double>(pl, v, s.kit + done, m, batch > 0, &ok);
+    }));
+    RETCHK(read_state<double>(pl, s));
     if (s.done) break;
-    len = pred.next(s, s.tol, 8);
+    len = pred.next(s, s.tol);
   }
   const int gb = grid_blocks(nv);
   if (s.pend)
@@ -1801,6 +1812,7 @@ int fh_plan_destroy(fh_plan* pl) {
   if (pl->spec) (void)hipFree(pl->spec);
   if (pl->partial) (void)hipFree(pl->partial);
   if (pl->st) (void)hipFree(pl->st);
+  if (pl->st_host) (void)hipHostFree(pl->st_host);
   if (pl->hist) (void)hipFree(pl->hist);
   if (pl->work) (void)hipFree(pl->work);
   drop_graphs(pl);
@@ -1908,7 +1920,8 @@ int fh_plan_create(int dim, const int* N, const double* Y, int physics, int prim
   const size_t spec_bytes = (size_t)pl->ncomp * pl->nh * sizeof(cpx<double>);
   if (hipMalloc(&pl->spec, spec_bytes) != hipSuccess ||
       hipMalloc(&pl->partial, (pl->partial_cap + kAuxDoubles) * sizeof(double)) != hipSuccess ||
-      hipMalloc(&pl->st, 2 * sizeof(CGState)) != hipSuccess)
+      hipMalloc(&pl->st, 2 * sizeof(CGState)) != hipSuccess ||
+      hipHostMalloc((void**)&pl->st_host, sizeof(CGState), hipHostMallocDefault) != hipSuccess)
     return bail(fail(FH_ERR_HIP, "hipMalloc plan buffers failed (out of device memory?)"));
   pl->aux = pl->partial + pl->partial_cap;
   pl->st_add = pl->st + 1;
@@ -2168,10 +2181,9 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
       if (every > 0) batch = std::min(batch, every - kit_host % every);
       if (cb_every > 0) batch = std::min(batch, cb_every - kit_host % cb_every);
       for (int k = 0; k < batch; ++k) RETCHK(enqueue_iteration<double>(pl, x, r, p, Ap, pl->coef64));
-      HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
-      HIPCHK(hipStreamSynchronize(pl->stream));
+      RETCHK(read_state(pl, s, nullptr, 0));
       kit_host = s.kit;
-      next_len = pred.next(s, s.tol, per_check);
+      next_len = pred.next(s, s.tol);
       if (s.done && x0_zero) {
         // x <- G x once at the end: the recurrence leaves x outside the range of G by its accumulated
         // rounding, which enters the energy (and the bound ordering) at first order; the projection
@@ -2238,17 +2250,18 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
     // (nr < delta * rmax, rmax the last true residual: after a pause, about the current norm)
     auto next_len = [&]() {
       const double rmax = s.pause ? std::sqrt(s.rr) : s.rmax;
-      len = pred.next(s, std::max(s.tol, s.delta * rmax), per_check);
+      len = pred.next(s, std::max(s.tol, s.delta * rmax));
     };
     for (;; ++batch) {
       if (fused) {
-        RETCHK(fused_batch<float>(pl, fv, s.kit, len, batch > 0, &fused));
+        RETCHK(run_batches(len, [&](int m, int done) {
+          return fused ? fused_batch<float>(pl, fv, s.kit + done, m, batch > 0, &fused) : (int)FH_OK;
+        }));
         if (!fused) pl->cg_defer = false;  // not covered: nothing was enqueued, use the general iteration
       }
       if (!fused)
         for (int k = 0; k < len; ++k) RETCHK(enqueue_iteration<float>(pl, xc, r, p, Ap, pl->coef32));
-      HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
-      HIPCHK(hipStreamSynchronize(pl->stream));
+      RETCHK(read_state<float>(pl, s));
       if (s.done) break;
       next_len();
       if (s.pause) RETCHK(update());
@@ -2258,7 +2271,6 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
     if (!(s.xfresh && !s.pend)) RETCHK(fold());
   }
   HIPCHK(hipEventRecord(pl->ev1, pl->stream));
-  HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
   HIPCHK(hipStreamSynchronize(pl->stream));
   float ms = 0.f;
   HIPCHK(hipEventElapsedTime(&ms, pl->ev0, pl->ev1));
@@ -3830,11 +3842,11 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
     hipLaunchKernelGGL(fh::k_cg_restart, dim3(1), dim3(256), 0, pl->stream, pl->st, pl->partial, gb, pl->hist, false);
     HIPCHK(hipGetLastError());
     for (int batch = 0;; ++batch) {
-      RETCHK(fused_pot_batch(pl, x, r, p, len, batch > 0));
-      HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
-      HIPCHK(hipStreamSynchronize(pl->stream));
+      RETCHK(run_batches(len, [&](int m, int) { return fused_pot_batch(pl, x, r, p, m, batch > 0); }));
+      const int nt = rt_pot_args(pl, p, r, nullptr).ntiles;
+      RETCHK(read_state(pl, s, pl->partial + pl->partial_cap / 2, nt <= kPotDefer ? nt : 0));
       if (s.done) break;
-      len = pred.next(s, s.tol, per_check);
+      len = pred.next(s, s.tol);
     }
     if (s.pend)
       hipLaunchKernelGGL(fh::k_fold_step, dim3(grid_blocks(2 * nh)), block, 0, pl->stream, 2 * nh, (double*)x,
@@ -3864,8 +3876,7 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
     };
     for (;;) {
       RETCHK(batch64());
-      HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
-      HIPCHK(hipStreamSynchronize(pl->stream));
+      RETCHK(read_state(pl, s, nullptr, 0));
       if (s.done) break;
     }
   } else {
@@ -3888,23 +3899,24 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
     const void* const key[5] = {xc, r, p, pl->coef32, pl->spec};
     for (int batch = 0;; ++batch) {
       bool ok = true;
-      RETCHK(run_batch(pl, 3, 0, len, key, batch > 0, &ok, [&](bool*) -> int {
-        for (int k = 0; k < len; ++k) {
-          int nb = 0;
-          RETCHK(pot_operator<float>(pl, p, r, Ap, re32, p, halt, &nb));
-          hipLaunchKernelGGL(fh::k_cg_alpha, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, pl->partial, nb);
-          hipLaunchKernelGGL((fh::pot::k_pot_update<float>), grid, block, 0, pl->stream, xc, r, p, Ap, g, pl->st,
-                             pl->partial);
-          hipLaunchKernelGGL(fh::k_cg_beta, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, pl->partial, gb);
-          HIPCHK(hipGetLastError());
-        }
-        return FH_OK;
+      RETCHK(run_batches(len, [&](int m, int) {
+        return run_batch(pl, 3, 0, m, key, batch > 0, &ok, [&](bool*) -> int {
+          for (int k = 0; k < m; ++k) {
+            int nb = 0;
+            RETCHK(pot_operator<float>(pl, p, r, Ap, re32, p, halt, &nb));
+            hipLaunchKernelGGL(fh::k_cg_alpha, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, pl->partial, nb);
+            hipLaunchKernelGGL((fh::pot::k_pot_update<float>), grid, block, 0, pl->stream, xc, r, p, Ap, g, pl->st,
+                               pl->partial);
+            hipLaunchKernelGGL(fh::k_cg_beta, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, pl->partial, gb);
+            HIPCHK(hipGetLastError());
+          }
+          return FH_OK;
+        });
       }));
-      HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
-      HIPCHK(hipStreamSynchronize(pl->stream));
+      RETCHK(read_state(pl, s, nullptr, 0));
       if (s.done) break;
       const double rmax = s.pause ? std::sqrt(s.rr) : s.rmax;
-      len = pred.next(s, std::max(s.tol, s.delta * rmax), per_check);
+      len = pred.next(s, std::max(s.tol, s.delta * rmax));
       if (s.pause) {
         hipLaunchKernelGGL(fh::k_fold_correction, dim3(fb), block, 0, pl->stream, 2 * nh, (double*)x, (float*)xc, false);
         RETCHK(pot_operator<double>(pl, x, nullptr, Ax, re, nullptr, nullptr, nullptr));
@@ -3933,7 +3945,6 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
     }
   }
   HIPCHK(hipEventRecord(pl->ev1, pl->stream));
-  HIPCHK(hipMemcpyAsync(&s, pl->st, sizeof(s), hipMemcpyDeviceToHost, pl->stream));
   HIPCHK(hipStreamSynchronize(pl->stream));
   float ms = 0.f;
   HIPCHK(hipEventElapsedTime(&ms, pl->ev0, pl->ev1));

@@ -706,8 +706,8 @@ static __global__ void k_cg_beta(CGState* st, const double* __restrict__ partial
   if (threadIdx.x == 0) finalize_beta(st, b);
 }
 
-// The deferred beta of a fused iteration on a small grid, at the end of a batch of iterations, so
-// that the host reads a finalised state (the same sum and decision as cg_fin_block).
+// The deferred beta of a fused iteration (the same sum and decision as cg_fin_block), where a kernel that
+// needs it has no block of its own to finalise it.
 static __global__ void k_cg_flush(CGState* st, const double* __restrict__ partial, int np) {
   if (st->halt || !st->bpend) return;
   const double rs = fixed_sum_partials(partial, np);
@@ -715,6 +715,24 @@ static __global__ void k_cg_flush(CGState* st, const double* __restrict__ partia
     finalize_beta(st, rs);
     st->bpend = 0;
   }
+}
+
+// End of a batch of iterations: the deferred beta (np partials, 0: none), then the state to `host`, pinned
+// memory that the host reads after the synchronisation (a copy to pageable memory is a kernel too, and a
+// staged one).
+static __global__ void k_cg_publish(CGState* st, const double* __restrict__ partial, int np, CGState* host) {
+  if (np && !st->halt && st->bpend) {
+    const double rs = fixed_sum_partials(partial, np);
+    if (threadIdx.x == 0) {
+      finalize_beta(st, rs);
+      st->bpend = 0;
+    }
+  }
+  __syncthreads();
+  static_assert(sizeof(CGState) % 8 == 0, "copied in 8-byte words");
+  const unsigned long long* src = reinterpret_cast<const unsigned long long*>(st);
+  unsigned long long* dst = reinterpret_cast<unsigned long long*>(host);
+  for (int i = threadIdx.x; i < (int)(sizeof(CGState) / 8); i += blockDim.x) dst[i] = src[i];
 }
 
 // 16-byte vector of T (4 floats or 2 doubles) for the streaming CG kernels.
