@@ -19,43 +19,88 @@ import torch
 from . import _native as nat
 
 
+class _Buffers:
+    """Where a call's float64 arrays live. For a theta on the library's GPU they are torch tensors lent to the
+    library (nothing travels through host memory, and torch's allocator gives the memory that a fresh
+    hipMalloc and hipFree per array would map and unmap): at 99^3 with gradient the four copies of 7.8 MB
+    to or from pageable memory and ten 23 MB allocations took 8 ms beside 25 ms of solves, what is left
+    takes 3 ms. Otherwise device arrays, filled and read through the host.
+
+    The library works on a stream of its own and every call has finished on return; sync() orders the
+    current torch stream (what filled an array, or used its memory before) ahead of such a call."""
+
+    def __init__(self, theta):
+        self.device = theta.device
+        self.lent = theta.is_cuda and theta.device.index == 0
+
+    def sync(self):
+        if self.lent:
+            torch.cuda.current_stream(self.device).synchronize()
+
+    def lend(self, t):
+        """A contiguous float64 tensor on the GPU as a device array that keeps it alive."""
+        v = nat.DeviceArray.borrow(t.data_ptr(), tuple(t.shape))
+        v._owner = t
+        return v
+
+    def array(self, shape, zero=False):
+        if self.lent:
+            return self.lend((torch.zeros if zero else torch.empty)(shape, dtype=torch.float64, device=self.device))
+        return nat.DeviceArray.zeros(shape) if zero else nat.DeviceArray(shape)
+
+    def put(self, t):
+        """The values of a tensor."""
+        if self.lent:
+            return self.lend(t.detach().to(self.device, torch.float64, copy=True).contiguous())
+        return nat.DeviceArray.from_host(t.detach().to('cpu', torch.float64).numpy())
+
+    def tensor(self, arr):
+        """An array of this call as a tensor on theta's device."""
+        return arr._owner if self.lent else torch.from_numpy(arr.to_host()).to(self.device)
+
+
+def _solve_unit_loads(theta, Y, tol, maxiter, precision):
+    """(buffers, plan, a, fields, iteration counts) of the d unit-load problems for a = exp(theta)."""
+    N = tuple(int(n) for n in theta.shape)
+    d = len(N)
+    buf = _Buffers(theta)
+    a = buf.put(torch.exp(theta.detach()))
+    plan = nat.Plan(N, np.asarray(Y, dtype=np.float64), 'scalar', 'primal')
+    B = buf.array((d,) + N)
+    EN = buf.array((d,) + N, zero=True)
+    fields = [buf.array((d,) + N, zero=True) for _ in range(d)]
+    buf.sync()
+    plan.set_coeff('iso', a)
+    kits = []
+    for iL, x in enumerate(fields):
+        E = np.zeros(d)
+        E[iL] = 1.
+        nat.add_constant(EN, -E)
+        plan.matvec(EN, B)
+        nat.add_constant(EN, E)  # back to exact zeros
+        info = plan.cg_solve(B, x, tol=tol, maxiter=maxiter, mode=precision)
+        if info['status'] != nat.FH_CG_OK:
+            raise FloatingPointError('CG breakdown')
+        nat.add_constant(x, E)
+        kits.append(info['kit'])
+    return buf, plan, a, fields, kits
+
+
 class UpperBound(torch.autograd.Function):
     """AH(theta) with a = exp(theta), scalar conductivity on an N grid of cell Y."""
 
     @staticmethod
     def forward(ctx, theta, Y, tol, maxiter, precision):
-        N = tuple(int(n) for n in theta.shape)
-        d = len(N)
-        a = torch.exp(theta.detach()).to('cpu', torch.float64).numpy()
-        plan = nat.Plan(N, np.asarray(Y, dtype=np.float64), 'scalar', 'primal')
-        plan.set_coeff('iso', a)
-        fields, kits = [], []
-        B = nat.DeviceArray((d,) + N)
-        for iL in range(d):
-            E = np.zeros(d)
-            E[iL] = 1.
-            EN = nat.DeviceArray.zeros((d,) + N)
-            nat.add_constant(EN, -E)
-            plan.matvec(EN, B)
-            x = nat.DeviceArray.zeros((d,) + N)
-            info = plan.cg_solve(B, x, tol=tol, maxiter=maxiter, mode=precision)
-            if info['status'] != nat.FH_CG_OK:
-                raise FloatingPointError('CG breakdown')
-            kits.append(info['kit'])
-            nat.add_constant(x, E)
-            fields.append(x)
-        AH = plan.energy_matrix(fields)
-        ctx.plan, ctx.fields = plan, fields
-        ctx.a_dev = nat.DeviceArray.from_host(a)
-        ctx.theta_device = theta.device
-        ctx.kits = kits
-        return torch.from_numpy(AH).to(theta.device)
+        ctx.buf, ctx.plan, ctx.a_dev, ctx.fields, ctx.kits = _solve_unit_loads(theta, Y, tol, maxiter, precision)
+        return torch.from_numpy(ctx.plan.energy_matrix(ctx.fields)).to(theta.device)
 
     @staticmethod
     def backward(ctx, gAH):
         W = gAH.detach().to('cpu', torch.float64).numpy()
-        g = ctx.plan.energy_gradient(ctx.fields, W, chain=ctx.a_dev)
-        return torch.from_numpy(g.to_host()).to(ctx.theta_device), None, None, None, None
+        out = ctx.buf.array(ctx.plan.N)
+        ctx.buf.sync()
+        g = ctx.plan.energy_gradient(ctx.fields, W, chain=ctx.a_dev, out=out)
+        return ctx.buf.tensor(g), None, None, None, None
 
 
 def upper_bound(theta, Y=None, tol=1e-10, maxiter=5000, precision='fp64'):
@@ -65,56 +110,30 @@ def upper_bound(theta, Y=None, tol=1e-10, maxiter=5000, precision='fp64'):
     return UpperBound.apply(theta, Y, tol, maxiter, precision)
 
 
-def _solve_unit_loads(theta, Y, tol, maxiter, precision):
-    N = tuple(int(n) for n in theta.shape)
-    d = len(N)
-    a = torch.exp(theta.detach()).to('cpu', torch.float64).numpy()
-    plan = nat.Plan(N, np.asarray(Y, dtype=np.float64), 'scalar', 'primal')
-    plan.set_coeff('iso', a)
-    fields = []
-    B = nat.DeviceArray((d,) + N)
-    for iL in range(d):
-        E = np.zeros(d)
-        E[iL] = 1.
-        EN = nat.DeviceArray.zeros((d,) + N)
-        nat.add_constant(EN, -E)
-        plan.matvec(EN, B)
-        x = nat.DeviceArray.zeros((d,) + N)
-        info = plan.cg_solve(B, x, tol=tol, maxiter=maxiter, mode=precision)
-        if info['status'] != nat.FH_CG_OK:
-            raise FloatingPointError('CG breakdown')
-        nat.add_constant(x, E)
-        fields.append(x)
-    return plan, a, fields
-
-
 class SolutionFields(torch.autograd.Function):
     """e (d, d) + N: e[i] = E_i + x_i for a = exp(theta); backward by adjoint CG solves."""
 
     @staticmethod
     def forward(ctx, theta, Y, tol, maxiter):
-        plan, a, fields = _solve_unit_loads(theta, Y, tol, maxiter, 'fp64')
-        ctx.plan, ctx.fields, ctx.tol, ctx.maxiter = plan, fields, tol, maxiter
-        ctx.a_dev = nat.DeviceArray.from_host(a)
-        ctx.theta_device = theta.device
-        return torch.from_numpy(np.stack([f.to_host() for f in fields])).to(theta.device)
+        ctx.buf, ctx.plan, ctx.a_dev, ctx.fields, _ = _solve_unit_loads(theta, Y, tol, maxiter, 'fp64')
+        ctx.tol, ctx.maxiter = tol, maxiter
+        return torch.stack([ctx.buf.tensor(f) for f in ctx.fields])  # a copy: the caller may write to it
 
     @staticmethod
     def backward(ctx, g):
-        plan = ctx.plan
-        g = g.detach().to('cpu', torch.float64).numpy()
-        adj = []
-        for i, f in enumerate(ctx.fields):
-            gi = nat.DeviceArray.from_host(np.ascontiguousarray(g[i]))
-            b = nat.DeviceArray(f.shape)
-            plan.project(gi, b)
-            lam = nat.DeviceArray.zeros(f.shape)
-            info = plan.cg_solve(b, lam, tol=ctx.tol, maxiter=ctx.maxiter, mode='fp64')
+        plan, buf = ctx.plan, ctx.buf
+        gi = [buf.put(v) for v in g.detach()]
+        b = [buf.array(f.shape) for f in ctx.fields]
+        adj = [buf.array(f.shape, zero=True) for f in ctx.fields]
+        out = buf.array(plan.N)
+        buf.sync()
+        for v, rhs, lam in zip(gi, b, adj):
+            plan.project(v, rhs)
+            info = plan.cg_solve(rhs, lam, tol=ctx.tol, maxiter=ctx.maxiter, mode='fp64')
             if info['status'] != nat.FH_CG_OK:
                 raise FloatingPointError('adjoint CG breakdown')
-            adj.append(lam)
-        grad = plan.field_gradient(ctx.fields, adj, chain=ctx.a_dev)
-        return torch.from_numpy(grad.to_host()).to(ctx.theta_device), None, None, None
+        grad = plan.field_gradient(ctx.fields, adj, chain=ctx.a_dev, out=out)
+        return buf.tensor(grad), None, None, None
 
 
 def solution_fields(theta, Y=None, tol=1e-10, maxiter=5000):
