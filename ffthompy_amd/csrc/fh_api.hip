@@ -1666,23 +1666,27 @@ void drop_graphs(fh_plan* pl) {
 
 // Number of CG iterations up to the next host synchronisation: what the convergence rate since the last
 // one predicts until the residual norm falls below `target` (the next stop or reliable-update threshold),
-// plus one, between 1 and the iterations done so far (8 to 64: a wrong prediction must not double the
-// work). An iteration enqueued past the stop returns at once on the halt flag but still dispatches its
-// grids (2-3 us each); a synchronisation costs 20 us and more. They are enqueued in batches of 8, 4, 2
-// and 1 (captured graphs, four lengths per kind of iteration): 135 x 135 fp64, 40 iterations: 1130 us
-// with a synchronisation and a copied state every 8 of them, 1050 us so.
+// plus one, between 1 and the iterations done so far (a wrong prediction must not double the work), at
+// most 8 to 64 by the size of the problem and never past the iteration limit. An iteration enqueued past
+// the stop returns at once on the halt flag but still dispatches its grids: 2-3 us a launch up to some
+// 10^5 values, 10 us at 225^3, where a synchronisation (20 us and more) costs less than one too many.
+// They are enqueued in batches of 8, 4, 2 and 1 (captured graphs, four lengths per kind of iteration):
+// 135 x 135 fp64, 40 iterations: 1130 us with a synchronisation and a copied state every 8 of them, 1050
+// us so.
 struct BatchPredictor {
+  const long long values;  // of one vector
   double nr_prev = -1.0;
   int kit_prev = 0;
   double rate = -1.0;
   int next(const CGState& s, double target) {
-    const int cap = std::min(64, std::max(8, s.kit));
+    const int most = values <= (1LL << 20) ? 64 : (values <= (1LL << 23) ? 16 : 8);
+    const int cap = std::max(1, std::min({most, std::max(8, s.kit), s.maxiter - s.kit}));
     const double nr = std::sqrt(s.rr);
     if (nr_prev > 0.0 && s.kit > kit_prev && nr > 0.0)
       rate = nr < nr_prev ? std::pow(nr / nr_prev, 1.0 / (double)(s.kit - kit_prev)) : -1.0;
     nr_prev = nr;
     kit_prev = s.kit;
-    if (!(rate > 0.0 && rate < 1.0) || !(target > 0.0) || !(nr > target)) return 8;
+    if (!(rate > 0.0 && rate < 1.0) || !(target > 0.0) || !(nr > target)) return std::min(8, cap);
     const double n = std::log(target / nr) / std::log(rate);
     return n < (double)cap ? std::min(cap, (int)std::ceil(n) + 1) : cap;
   }
@@ -1717,7 +1721,7 @@ static int cg_fused64(fh_plan* pl, const double* b, double* x, bool x0_zero, CGS
     HIPCHK(hipMemcpyAsync(xw, x, (size_t)nv * sizeof(double), hipMemcpyDeviceToDevice, pl->stream));
   }
   RETCHK(enqueue_true_residual<double>(pl, b, x, p0, r, x0_zero));
-  BatchPredictor pred;
+  BatchPredictor pred{nv};
   int len = 8;
   pl->last_graph_batches = 0;
   for (int batch = 0;; ++batch) {
@@ -2172,7 +2176,7 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
     const int cb_every = pl->it_fn ? pl->it_every : 0;
     int cb_last = 0;
     int kit_host = 0;
-    BatchPredictor pred;
+    BatchPredictor pred{nv};
     int next_len = per_check;
     for (;;) {
       // batches end on the logged / called-back iterations (multiples of every, cb_every), at
@@ -2244,7 +2248,7 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
     // fused iterations is captured once as a HIP graph and replayed (fused_batch)
     int batch = 0;
     pl->last_graph_batches = 0;
-    BatchPredictor pred;
+    BatchPredictor pred{nv};
     int len = per_check;
     // after a synchronisation: the next threshold is the stop test or the reliable update
     // (nr < delta * rmax, rmax the last true residual: after a pause, about the current norm)
@@ -3830,7 +3834,7 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
                      nullptr);
   const int* halt = &pl->st->halt;
   const int per_check = 8;
-  BatchPredictor pred;
+  BatchPredictor pred{2 * nh};
   int len = per_check;
   if (fused) {
     // the plan's own iterate (captured batches keep its address) in the place of A p
