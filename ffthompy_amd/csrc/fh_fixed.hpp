@@ -213,20 +213,31 @@ struct FxShape {
   // full the last wavefront of a workgroup is); strided passes: columns per tile.
   static constexpr int NPROJ = 4, NCOLS = 2;
   static constexpr int proj_f(int v) {
-    constexpr int c32a[NPROJ] = {4, 6, 5, 7}, c32b[NPROJ] = {16, 8, 12, 24}, c32c[NPROJ] = {32, 16, 24, 48};
-    constexpr int c64a[NPROJ] = {4, 2, 3, 6}, c64b[NPROJ] = {8, 4, 6, 12}, c64c[NPROJ] = {16, 8, 12, 24};
+    constexpr int c32a[NPROJ] = {6, 4, 5, 7}, c32b[NPROJ] = {8, 16, 12, 24}, c32c[NPROJ] = {16, 32, 24, 48};
+    constexpr int c64a[NPROJ] = {3, 2, 4, 6}, c64b[NPROJ] = {6, 4, 8, 12}, c64c[NPROJ] = {12, 8, 16, 24};
     if (sizeof(T) == 4) return FP::TPP >= 16 ? c32a[v] : (FP::TPP >= 8 ? c32b[v] : c32c[v]);
     return FP::TPP >= 16 ? c64a[v] : (FP::TPP >= 8 ? c64b[v] : c64c[v]);
   }
   static constexpr int cols_p(int v) { return v == 0 ? P : (P >= 2 ? P / 2 : P); }
-  // contiguous-axis passes: rows per workgroup (even); variant 1 takes 3/2 as many rows in single
-  // precision and 1/2 as many in double, variant 2 3/4 as many, which also changes how full the
-  // last wavefront is (TPP * (rpb/2) * NC threads: 243 points, 3 components: 8 rows 324 threads
-  // in 6 wavefronts, 12 rows 486 in 8, 6 rows 243 in 4, 4 rows 162 in 3) and how many workgroups
-  // share a CU's LDS
+  // contiguous-axis passes: rows per workgroup (even), RPB, half or one and a half of it, or 3/4, which
+  // changes how full the last wavefront is (TPP * (rpb/2) * NC threads: 243 points, 3 components: 8 rows 324
+  // threads in 6 wavefronts, 12 rows 486 in 8, 6 rows 243 in 4, 4 rows 162 in 3) and how many workgroups
+  // share a CU's LDS. Table entry 0 covers every coefficient (in double precision with direct loads), the
+  // others none and isotropic with 2 or 3 components, staged. rows_index: schedule variant v as a table
+  // entry; by default 3/2 of RPB at 225 points and more and 3/4 below in single precision with up to three
+  // components (six: RPB, 243^3 elasticity 777 against 864 us), 3/4 in double, staged where it can be.
+  // Against defaults of RPB rows and projection tiles of 4 (8, 16) points, per operator application: double
+  // 243^3 763 -> 671 us, 225^3 662 -> 555, 125^3 104 -> 95, 243 x 135 x 225 393 -> 319, 243 x 81 x 99 112
+  // -> 100, 243^3 elasticity 1872 -> 1564; single 243^3 337 -> 320 (40 CG iterations 24.6 -> 23.2 ms), 225^3
+  // 254 -> 255 (20.8 -> 19.7 ms), 243 x 243 x 135 188 -> 183.
   static constexpr int NROWS = 3;
-  static constexpr int rows_rpb(int v) {
-    return v == 0 ? RPB : (v == 1 ? (sizeof(T) == 4 ? RPB / 2 * 3 : RPB / 2) : RPB / 4 * 3);
+  static constexpr int rows_rpb(int e) {
+    if (sizeof(T) == 4) return e == 0 ? RPB : (e == 1 ? RPB / 2 * 3 : RPB / 4 * 3);
+    return e == 1 ? RPB / 2 : RPB / 4 * 3;
+  }
+  static constexpr int rows_index(int v, int nc) {
+    const int best = nc == 6 ? 0 : (sizeof(T) == 4 && FP::TPP >= 16 ? 1 : 2);
+    return v == 0 ? best : (v == best ? 0 : v);
   }
 };
 
