@@ -103,7 +103,7 @@ int fh_plan_use_generic(fh_plan* plan, int generic);
  * with fused = 0, they use the operator form. */
 int fh_plan_set_cg_variant(fh_plan* plan, int fused);
 
-/* Mixed-precision CG with the fused iteration: enable = 1 (default) replays batches of
+/* CG with fused iterations and mixed potential solves: enable = 1 (default) replays batches of
  * iterations from a HIP graph captured on the plan's stream (kernel nodes only, rebuilt when a
  * work buffer moves); 0 launches every kernel directly. Same arithmetic either way.
  * fh_last_solve_graph_batches: batches of the last solve that ran from the graph.
@@ -353,8 +353,8 @@ int fh_matvec_profile(fh_plan* plan, int dtype, const void* x, void* y, int nrep
  * (0..3) sets the frequency points per tile of the projection pass (forward FFT along the
  * outermost axis, G(xi), inverse FFT), which also sets the threads per workgroup; cols_variant (0..1) the columns per tile of the other strided
  * passes (3-D); rows_variant (0..2) the grid rows per workgroup of the contiguous-axis passes
- * (variant 1: 3/2 as many in single precision, 1/2 as many in double; variant 2: 3/4 as many;
- * scalar plans, isotropic or no coefficient). Every variant computes the same values (the same
+ * (0, the default, the fastest on the grids measured, which depends on the axis length, the arithmetic and the
+ * number of components; scalar plans, isotropic or no coefficient). Every variant computes the same values (the same
  * transforms per pencil); only speed differs. Variant 0 is the default.
  * fh_plan_autotune times every variant on this plan (3 interleaved rounds of nrep matvecs of x
  * into y per variant, each pass timed by its own HIP events, as fh_matvec_profile; a variant's
@@ -376,8 +376,8 @@ int fh_plan_autotune(fh_plan* plan, int dtype, const void* x, void* y, int nrep,
  * Y[2s] x Y[2s+1] (NULL: unit cells), unit loads E = e1, e2, CG (ffthompy/general/solver.py:80-139)
  * on the primal (G1, a) and dual (G2, 1/a) problems, and the bounds of
  * ffthompy/postprocess.py:53-70: upper = <a e_i, e_j>, lower = inv(<a^-1 e_i, e_j>).
- * All samples are solved by one persistent kernel (one workgroup per sample and primal/dual
- * task, CG state on the device), launched from a captured HIP graph. */
+ * All samples are solved by one persistent kernel (one workgroup per sample, primal/dual
+ * problem and, up to 2048 samples, unit load; CG state on the device), launched from a captured HIP graph. */
 int fh_batch_create(int nsamples, const int* dims, const double* Y, fh_batch** out);
 int fh_batch_destroy(fh_batch* batch);
 /* a: host fp64, the samples' voxel values concatenated, each in C order with origin at
