@@ -607,6 +607,7 @@ int rt_cols(fh_plan* pl, int mode, int axis, int nc, const cpx<T>* src, cpx<T>* 
   a.halt = halt;
   if (fin) a.fin = *fin;
   a.total = (long long)nc * pl->nh;
+  if (a.total * (long long)sizeof(cpx<T>) >= fh::rt::kSpan) return fail(FH_ERR_STATE, "strided pass: spectrum too large");
   a.cs = (int)pl->nh;
   int nthr;
   size_t lds;
@@ -665,7 +666,15 @@ int rt_operator_front(fh_plan* pl, const T* x, int kind, const T* coef, const in
   return rt_middle<T>(pl, spec, g, halt);
 }
 
-// Forward transform of A(x) x (kind COEF_NONE: of x) into xhat, every component in one launch per pass.
+// Components that one launch of the strided passes takes: their resource spans all of them and has to stay
+// below 2 GiB (fh::rt::kSpan), which the plan's own components do (make_config); 36 is the largest tensor field.
+template <typename T>
+int rt_group(const fh_plan* pl) {
+  return (int)std::min<long long>(36, (fh::rt::kSpan - 1) / (pl->nh * (long long)sizeof(cpx<T>)));
+}
+
+// Forward transform of A(x) x (kind COEF_NONE: of x) into xhat, every component (at most rt_group) in one
+// launch per pass.
 template <typename T>
 int rt_forward(fh_plan* pl, int nc, const T* x, const T* coef, int kind, cpx<T>* xhat) {
   fh::rt::FwdArgs<T> a{};
@@ -898,7 +907,13 @@ static int matvec_impl(fh_plan* pl, int dtype, const void* x, void* y, bool with
 
 template <typename T>
 static int rfftn_impl(fh_plan* pl, int ncomp, const T* x, cpx<T>* xhat) {
-  if (rt_on<T>(pl)) return rt_forward<T>(pl, ncomp, x, nullptr, fh::COEF_NONE, xhat);  // the 'r' layout itself
+  if (rt_on<T>(pl)) {  // the 'r' layout itself
+    const int most = rt_group<T>(pl);
+    for (int c0 = 0; c0 < ncomp; c0 += most)
+      RETCHK(rt_forward<T>(pl, std::min(most, ncomp - c0), x + (size_t)c0 * pl->n, nullptr, fh::COEF_NONE,
+                           xhat + (size_t)c0 * pl->nh));
+    return FH_OK;
+  }
   const GParams g = make_gparams(pl, 1.0, 1);
   for (int c = 0; c < ncomp; ++c) {
     cpx<T>* out = xhat + (size_t)c * pl->nh;

@@ -180,9 +180,10 @@ struct TangleAcc {
 };
 
 // HBM through a buffer resource: element e of pencil q at byte e * es + qoff, qoff given by the kernel
-// (kDead for a pencil outside the tile). The resource is below 2 GiB, so kDead plus any step is out of
-// range and does not wrap.
+// (kDead for a pencil outside the tile). The resource is below 2 GiB (kSpan, checked by the host), so kDead
+// plus any step is out of range and does not wrap.
 constexpr unsigned kDead = 0x80000000u;
+static_assert(kDead == kSpan, "dead lanes sit past every resource");
 
 template <typename T>
 struct BufAcc {

@@ -143,6 +143,10 @@ constexpr int round64(long long n) { return (int)((n + 63) / 64 * 64); }
 // -> 28.4, 60^3 single 22.0 -> 21.1; no grid measured slower).
 constexpr int roundw(long long n) { return n <= 128 ? round64(n) : (int)((n + 255) / 256 * 256); }
 
+// What a pass reaches through one buffer resource stays below this: lanes without work take byte offsets from
+// kDead = 2^31 on, which a larger resource would hold.
+constexpr long long kSpan = 1LL << 31;
+
 constexpr size_t kLdsBytes = 160 * 1024;
 constexpr size_t kLdsUse = kLdsBytes - 2048;  // static LDS of the kernels and rounding
 

@@ -56,7 +56,7 @@ Config make_config(size_t rb, int n0, int n1, int n2, int nc) {
   if (!div_exact((long long)n1 * g.n2h, g.n2h)) return c;
   g.dn2 = make_div(n2);
   g.dn2h = make_div(g.n2h);
-  if ((unsigned long long)nc * g.nh * 2 * rb >= (1ULL << 31)) return c;  // buffer offsets (see kDead)
+  if (nc * g.nh * 2 * (long long)rb >= kSpan) return c;
   // Plane mode (the whole plane of one component in LDS) for every compiled plane (135^3: 114 us against
   // 130 us of row mode in double, 71 against 85 in single precision). A plane of other lengths runs the
   // schedule-driven kernel: it wins while one round of workgroups covers the chip (63 x 81 x 105, 189
@@ -105,7 +105,7 @@ Config make_config(size_t rb, int n0, int n1, int n2, int nc) {
 bool pad_config(int L, int es, long long outer, PadArgs* a, unsigned* nblk, int* nthr, size_t* lds) {
   a->ax = plan_axis(L);
   a->es = es;
-  if (!a->ax.nst || (unsigned long long)L * es * 16 >= (1ULL << 31)) return false;
+  if (!a->ax.nst || (long long)L * es * 16 >= kSpan) return false;
   if (!pick_cols(a->ax, 1, 8, es, outer, 3, 2, 1024, 48 * 1024, &a->lf, nthr, &a->tpp, lds)) return false;
   a->ntiles = (es + (1 << a->lf) - 1) >> a->lf;
   a->dtiles = make_div(a->ntiles);
