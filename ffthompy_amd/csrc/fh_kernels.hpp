@@ -264,6 +264,14 @@ __device__ __forceinline__ void finalize_alpha(CGState* st, double psum) {
   }
 }
 
+// alpha of a fused iteration, whose first pass has added the step pending before it to the solution: that step
+// is done, and this iteration's is pending instead, or none is at a breakdown.
+__device__ __forceinline__ void cg_step_known(CGState* st, double psum) {
+  finalize_alpha(st, psum);
+  if (st->pend) st->xfresh = 0;  // the correction was written
+  st->pend = st->status == 0 ? 1 : 0;
+}
+
 // The step that <r,r> = rsum (unscaled) makes: rr_new, beta = rr_new / rr, the iteration count,
 // the norm and the stop decisions. One function, so that every kernel that evaluates it from the
 // same sum takes the same decision.
@@ -358,9 +366,7 @@ __device__ __forceinline__ void cg_fin_block(const CgFin& f) {
   }
   const double ps = fixed_sum_partials(f.p1, f.n1);
   if (threadIdx.x == 0) {
-    finalize_alpha(st, ps);
-    if (st->pend) st->xfresh = 0;  // this iteration's forward pass wrote the correction
-    st->pend = st->status == 0 ? 1 : 0;
+    cg_step_known(st, ps);
   }
 }
 
@@ -691,9 +697,7 @@ static __global__ void k_cg_alpha(CGState* st, const double* __restrict__ partia
   for (int i = threadIdx.x; i < np; i += blockDim.x) acc += partial[i];
   const double b = block_sum(acc);
   if (threadIdx.x == 0) {
-    finalize_alpha(st, b);
-    if (st->pend) st->xfresh = 0;  // this iteration's forward pass wrote the correction
-    st->pend = st->status == 0 ? 1 : 0;
+    cg_step_known(st, b);
   }
 }
 

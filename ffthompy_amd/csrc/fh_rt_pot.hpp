@@ -112,7 +112,7 @@ __global__ void __launch_bounds__(512) k_pot(PotArgs A) {
         ps = fixed_sum_partials(A.p1, A.np1);
         const double pAp = ps * A.st->inv_nvox;
         if (!(pAp > 0.0) || !isfinite(pAp)) {  // breakdown: no workgroup changes r
-          if (blockIdx.x == 0 && tid == 0) finalize_alpha(A.st, ps);
+          if (blockIdx.x == 0 && tid == 0) cg_step_known(A.st, ps);
           return;
         }
         alp = T(A.st->rr / pAp);
@@ -174,11 +174,7 @@ __global__ void __launch_bounds__(512) k_pot(PotArgs A) {
     if (step_r && blockIdx.x == 0 && tid == 0) {
       // the other workgroups read none of these
       CGState* st = A.st;
-      if (A.np1) {
-        finalize_alpha(st, ps);
-        if (st->pend) st->xfresh = 0;  // the pass before wrote the correction
-        st->pend = 1;
-      }
+      if (A.np1) cg_step_known(st, ps);
       if (A.defer_beta) st->bpend = 1;
     }
   }
