@@ -636,8 +636,7 @@ int rt_cols(fh_plan* pl, int mode, int axis, int nc, const cpx<T>* src, cpx<T>* 
   a.ntiles = (a.nf + (1 << a.lf) - 1) >> a.lf;
   a.dP = fh::rt::make_div((long long)ncf << a.lf);
   a.dtiles = fh::rt::make_div(a.ntiles);
-  const long long nb = outer * a.ntiles;
-  if (nb > 0x7fffffffLL || (mode != 2 && nb * a.ntiles >= (1LL << 32))) return fail(FH_ERR_UNSUPPORTED, "grid too large");
+  const long long nb = outer * a.ntiles;  // at most a.total, below 2^28
   return rt_result(fh::rt::launch_cols<T>(nc, mode, a, (unsigned)nb, nthr, lds, rt_launch(pl)), "strided pass");
 }
 

@@ -138,6 +138,12 @@ __device__ __forceinline__ int quot(int x, const Div d) {
   return d.d == 1 ? x : (int)__umulhi((unsigned)x, d.m);
 }
 
+// x / d for any x, d below 2^31, where the multiply-high alone is one too large at times (x * d >= 2^32).
+__device__ __forceinline__ int quot_any(int x, const Div d) {
+  const int q = quot(x, d);
+  return q - ((unsigned)q * d.d > (unsigned)x);
+}
+
 // ---- accessors: at(q, e, de) is element e of pencil q; get(j) / put(j, v) element e + j de -----------
 
 // LDS tile, element e of pencil q at e * es + q
@@ -684,7 +690,8 @@ __global__ void __launch_bounds__(512) k_cols(ColArgs<T> A) {
   const int L = CL > 0 ? CL : ax.L;
   cpx<T>* twl = s + L * P;
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
-  const int o = MODE == 2 ? 0 : quot(lin, A.dtiles), tile = lin - o * A.ntiles;
+  // a flat grid's tiles along the outermost axis, times its slabs, pass the range of quot()
+  const int o = MODE == 2 ? 0 : quot_any(lin, A.dtiles), tile = lin - o * A.ntiles;
   const int f0 = tile << lf;
   const int nf = min(F, A.nf - f0);
   for (int e = tid; e < L; e += nthr) twl[e] = A.tw[e];

@@ -40,3 +40,35 @@ def test_transform_of_more_than_two_gib(dt, ct, nc):
     for c in range(nc):
         plan.rfftn(part(x, c, (1,) + N), one, 1)
         assert np.array_equal(part(X, c, Nh).to_host(), one.to_host()[0]), c
+
+
+@pytest.mark.parametrize('N,nc', [((2, 2000, 2000), 1), ((2, 2000, 2000), 3), ((16, 1500, 1500), 1)])
+def test_transforms_of_flat_grids(N, nc):
+    """More tiles along the outermost axis (125125 of 16 points in double, 62563 of 32 in single precision at
+    2 x 2000 x 2000) than a multiply-high alone splits into slabs."""
+    print('case flat transforms', N, nc, flush=True)
+    rng = np.random.default_rng(65)
+    plan = nat.Plan(N, np.ones(len(N)))
+    Nh = N[:-1] + (N[-1] // 2 + 1,)
+    x = rng.standard_normal((nc,) + N)
+    ref = np.fft.rfftn(x, axes=tuple(range(1, x.ndim)))
+    for dt, ct, tol in ((np.float64, np.complex128, 1e-12), (np.float32, np.complex64, 2e-5)):
+        X = plan.rfftn(nat.DeviceArray.from_host(x.astype(dt)), nat.DeviceArray((nc,) + Nh, ct), nc)
+        assert rel(X.to_host(), ref) < tol, dt
+        z = plan.irfftn(X, nat.DeviceArray((nc,) + N, dt), nc)
+        assert rel(z.to_host(), x) < tol, dt
+
+
+def test_potential_solve_of_a_flat_grid():
+    """Iterates of the fp64 solve against the generic kernels (tolerance as in test_gpu_rt_potential.py)."""
+    N = (2, 2000, 2000)
+    print('case flat potential', N, flush=True)
+    plan = nat.Plan(N, np.ones(3))
+    plan.set_coeff('iso', np.exp(0.5 * np.random.default_rng(66).standard_normal(N)))
+    out = []
+    for generic in (True, False):
+        plan.use_generic(generic)
+        Fu, info = plan.potential_solve(np.array([1., 0.5, 0.2]), 1e-11, 4, mode='fp64')
+        out.append((Fu.to_host(), info['kit'], info['status']))
+    assert out[0][1:] == out[1][1:] == (4, nat.FH_CG_OK)
+    assert rel(out[1][0], out[0][0]) <= 1e-11
