@@ -122,16 +122,21 @@ class SolutionFields(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         plan, buf = ctx.plan, ctx.buf
-        gi = [buf.put(v) for v in g.detach()]
-        b = [buf.array(f.shape) for f in ctx.fields]
-        adj = [buf.array(f.shape, zero=True) for f in ctx.fields]
-        out = buf.array(plan.N)
-        buf.sync()
-        for v, rhs, lam in zip(gi, b, adj):
+        g = g.detach()
+        rhs = buf.array(ctx.fields[0].shape)
+        adj = []
+        for i, f in enumerate(ctx.fields):  # one load's gradient and right-hand side at a time
+            v = buf.put(g[i])
+            lam = buf.array(f.shape, zero=True)
+            buf.sync()
             plan.project(v, rhs)
             info = plan.cg_solve(rhs, lam, tol=ctx.tol, maxiter=ctx.maxiter, mode='fp64')
             if info['status'] != nat.FH_CG_OK:
                 raise FloatingPointError('adjoint CG breakdown')
+            adj.append(lam)
+        v = rhs = None
+        out = buf.array(plan.N)
+        buf.sync()
         grad = plan.field_gradient(ctx.fields, adj, chain=ctx.a_dev, out=out)
         return buf.tensor(grad), None, None, None
 
