@@ -266,15 +266,15 @@ struct fh_plan {
   bool defer_ok = true;          // fused iteration: alpha/beta inside the passes on small grids
   bool cg_defer = false;         // this solve runs the deferred alpha/beta
   CGState* st_host = nullptr;    // pinned copy of the CG state (k_cg_publish)
-  int pub_nb2[2] = {0, 0};       // the same of the last iteration enqueued or captured, fp64 and fp32
-  int defer_nb2 = 0;             // workgroups of the fused inverse row pass (its partials)
+  // partial sums of a deferred beta (workgroups of the inverse pass), fp64 and fp32, as of the last iteration
+  // enqueued or captured: kept from solve to solve, since a solve may start with captured batches
+  int beta_parts[2] = {0, 0};
   hipEvent_t prof_t0 = nullptr, prof_t1 = nullptr;  // matvec profile: events of the next launch
   int banded = 0;                // 1: projection restricted to |k_a| <= band[a] (view axes)
   int band[3] = {0, 0, 0};
   double op_scale = 1.0;         // factor of the operator G A (not of the bare projection)
-  // fused mixed CG: a batch of iterations captured once as a HIP graph, replayed per batch
-  // captured batches of 1, 2, 4, 8 iterations, by length, kind (0 fp64, 1 fp32, 2 and 3 the
-  // same of the potential formulation) and the direction buffer that the batch starts from
+  // batches of 1, 2, 4, 8 iterations, captured once as HIP graphs and replayed, by length, kind (0 fp64,
+  // 1 fp32, 2 and 3 the same of the potential formulation) and the direction buffer that the batch starts from
   hipGraphExec_t it_exec[9][4][2] = {};
   const void* it_key[4][5] = {};  // buffers the captured batches were built for, by kind
   bool it_graph_off = false;     // capture failed on this plan: direct launches from then on
@@ -1038,7 +1038,7 @@ static int enqueue_fused_rt(fh_plan* pl, T* xc, T* r, T* pin, T* pout, const T* 
   b.halt = halt;
   RETCHK(rt_inv<T>(pl, b, pl->ncomp, nullptr));
   if (defer) {
-    pl->pub_nb2[sizeof(T) == 8 ? 0 : 1] = pl->defer_nb2 = nb;
+    pl->beta_parts[sizeof(T) == 8 ? 0 : 1] = nb;
   } else {
     hipLaunchKernelGGL(fh::k_cg_beta, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, part2, nb);
     HIPCHK(hipGetLastError());
@@ -1062,7 +1062,7 @@ static int enqueue_fused_iteration(fh_plan* pl, float* xc, float* r, float* p, c
   fh::LaunchCtx ctx = make_ctx<float>(pl);
   if (defer) {
     ctx.bpart = part2;
-    ctx.bnp = pl->defer_nb2;
+    ctx.bnp = pl->beta_parts[1];
   }
   int nb = 0;
   int rr = fh::fixed_rows_fwd<float>(ctx, nc, p, coef, pl->coef_kind, spec, halt, r, pl->st, xc, part1,
@@ -1078,7 +1078,7 @@ static int enqueue_fused_iteration(fh_plan* pl, float* xc, float* r, float* p, c
   bool first_done = false;
   {
     fh::LaunchCtx cf = make_ctx<float>(pl);
-    cf.fin = fh::CgFin{pl->st, part1, defer ? part2 : nullptr, nb, defer ? pl->defer_nb2 : 0};
+    cf.fin = fh::CgFin{pl->st, part1, defer ? part2 : nullptr, nb, defer ? pl->beta_parts[1] : 0};
     const int rf = pl->n0 > 1 ? fh::fixed_cols<float>(cf, -1, 1, nc, spec, halt)
                               : fh::fixed_cols_g<float>(cf, 1, nc, spec, g, halt);
     if (rf != 0) {
@@ -1087,7 +1087,7 @@ static int enqueue_fused_iteration(fh_plan* pl, float* xc, float* r, float* p, c
     } else {
       // no fixed kernel on this axis: finalise with the one-workgroup kernels
       if (defer)
-        hipLaunchKernelGGL(fh::k_cg_flush, dim3(1), dim3(32), 0, pl->stream, pl->st, part2, pl->defer_nb2);
+        hipLaunchKernelGGL(fh::k_cg_flush, dim3(1), dim3(32), 0, pl->stream, pl->st, part2, pl->beta_parts[1]);
       hipLaunchKernelGGL(fh::k_cg_alpha, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, part1, nb);
     }
   }
@@ -1106,7 +1106,7 @@ static int enqueue_fused_iteration(fh_plan* pl, float* xc, float* r, float* p, c
   if (rr == 0) return fail(FH_ERR_STATE, "fused rows inverse unavailable");
   RETCHK(fixed_result(rr, "rows inverse (fused)"));
   if (defer)
-    pl->pub_nb2[1] = pl->defer_nb2 = nb2;
+    pl->beta_parts[1] = nb2;
   else
     hipLaunchKernelGGL(fh::k_cg_beta, dim3(1), dim3(kFinThreads), 0, pl->stream, pl->st, part2, nb2);
   HIPCHK(hipGetLastError());
@@ -1125,7 +1125,7 @@ static int read_state(fh_plan* pl, CGState& s, const double* part, int np) {
 // The same for a solve on the plan's operator in precision T.
 template <typename T>
 static int read_state(fh_plan* pl, CGState& s) {
-  return read_state(pl, s, pl->partial + kDeferMax, pl->cg_defer ? pl->pub_nb2[sizeof(T) == 8 ? 0 : 1] : 0);
+  return read_state(pl, s, pl->partial + kDeferMax, pl->cg_defer ? pl->beta_parts[sizeof(T) == 8 ? 0 : 1] : 0);
 }
 
 // Vectors of a fused solve: the correction (or, in fp64, the iterate), the residual and the two
@@ -1728,7 +1728,6 @@ static int cg_fused64(fh_plan* pl, const double* b, double* x, bool x0_zero, CGS
   double* p0 = r + nvp;
   const FusedVecs<double> v{xw, r, {p0, two ? p0 + nvp : p0}, pl->coef64};
   pl->cg_defer = defer_applies<double>(pl);
-  pl->defer_nb2 = 0;
   if (x0_zero) {
     HIPCHK(hipMemsetAsync(xw, 0, (size_t)nv * sizeof(double), pl->stream));
   } else {
@@ -2232,7 +2231,6 @@ int fh_cg_solve(fh_plan* pl, int mode, const void* b_, void* x_, double tol, int
     // fused iterations where the fixed-length kernels cover the plan (isotropic coefficient)
     bool fused = pl->fused_cg && pl->op_scale == 1.0;  // the fused step assumes an unscaled G
     pl->cg_defer = fused && defer_applies<float>(pl);
-    pl->defer_nb2 = 0;
     const int gb = grid_blocks(nv);
     // coupled coefficients read every component's old direction: two direction buffers in turn
     const bool two = rt_on<float>(pl) && pl->coef_kind != fh::COEF_ISO;
