@@ -210,33 +210,37 @@ struct FxShape {
   static constexpr int RPB = (FP::TPP >= 16) ? 8 : (FP::TPP >= 8 ? 16 : 32);
   // Schedule variants a plan can select (fh_plan_set_schedule / fh_plan_autotune); variant 0 is
   // the default. Projection pass: frequency points per tile (TPP*F*NC threads, so F also sets how
-  // full the last wavefront of a workgroup is); strided passes: columns per tile.
+  // full the last wavefront of a workgroup is); strided passes: columns per tile. Defaults by threads per
+  // pencil, the fastest or within a few percent over 5 .. 243 x 63 x 81 and x 225 x 225, three and six
+  // components (double precision: 135 x 225 x 225 57 us with 4 points, 70 with 8, 89 with 6; 99 x 225 x 225
+  // 41, 47, 38; 25 x 225 x 225 elasticity 21 with 8, 23 with 16, 28 with 12; 105 x 63 x 81 elasticity 16.7 with 4,
+  // 17.8 with 3; 243 x 225 x 225 131 with 3, 142 with 4; single: 105 x 225 x 225 25 with 4, 28 with 6;
+  // 243 x 225 x 225 50 with 6, 60 with 4).
   static constexpr int NPROJ = 4, NCOLS = 2;
   static constexpr int proj_f(int v) {
-    constexpr int c32a[NPROJ] = {6, 4, 5, 7}, c32b[NPROJ] = {8, 16, 12, 24}, c32c[NPROJ] = {16, 32, 24, 48};
-    constexpr int c64a[NPROJ] = {3, 2, 4, 6}, c64b[NPROJ] = {6, 4, 8, 12}, c64c[NPROJ] = {12, 8, 16, 24};
-    if (sizeof(T) == 4) return FP::TPP >= 16 ? c32a[v] : (FP::TPP >= 8 ? c32b[v] : c32c[v]);
-    return FP::TPP >= 16 ? c64a[v] : (FP::TPP >= 8 ? c64b[v] : c64c[v]);
+    constexpr int f32[4][NPROJ] = {{6, 4, 5, 7}, {4, 6, 5, 7}, {8, 16, 12, 24}, {16, 32, 24, 48}};
+    constexpr int f64[5][NPROJ] = {{3, 2, 4, 6}, {4, 2, 3, 6}, {4, 6, 8, 12}, {8, 12, 16, 24}, {12, 8, 16, 24}};
+    constexpr int c = FP::TPP >= 24 ? 0 : (FP::TPP >= 16 ? 1 : (FP::TPP >= 8 ? 2 : 3));
+    return sizeof(T) == 4 ? f32[c][v] : f64[c == 3 && FP::TPP < 5 ? 4 : c][v];
   }
   static constexpr int cols_p(int v) { return v == 0 ? P : (P >= 2 ? P / 2 : P); }
   // contiguous-axis passes: rows per workgroup (even), RPB, half or one and a half of it, or 3/4, which
   // changes how full the last wavefront is (TPP * (rpb/2) * NC threads: 243 points, 3 components: 8 rows 324
   // threads in 6 wavefronts, 12 rows 486 in 8, 6 rows 243 in 4, 4 rows 162 in 3) and how many workgroups
-  // share a CU's LDS. Table entry 0 covers every coefficient (in double precision with direct loads), the
-  // others none and isotropic with 2 or 3 components, staged. rows_index: schedule variant v as a table
-  // entry; by default 3/2 of RPB at 225 points and more and 3/4 below in single precision with up to three
-  // components (six: RPB, 243^3 elasticity 777 against 864 us), 3/4 in double, staged where it can be.
-  // Against defaults of RPB rows and projection tiles of 4 (8, 16) points, per operator application: double
-  // 243^3 763 -> 671 us, 225^3 662 -> 555, 125^3 104 -> 95, 243 x 135 x 225 393 -> 319, 243 x 81 x 99 112
-  // -> 100, 243^3 elasticity 1872 -> 1564; single 243^3 337 -> 320 (40 CG iterations 24.6 -> 23.2 ms), 225^3
-  // 254 -> 255 (20.8 -> 19.7 ms), 243 x 243 x 135 188 -> 183.
+  // share a CU's LDS. Table entry 0 (RPB rows) covers every coefficient (in double precision with direct loads),
+  // the others none and isotropic with 2 or 3 components, staged. rows_index: schedule variant v as a table
+  // entry; by default entry 0 with six components, else 3/4 of RPB, but 3/2 in single precision at 125, 225 and
+  // 243 points and half in double precision at 75 and 135. Forward + inverse rows, against RPB rows (double
+  // precision: direct): double 225 x 243 x 243 326 -> 263 us, 243 x 135 x 225 195 -> 140, 225 x 243 x 135
+  // 208 -> 144 (3/4: 164), 225 x 243 x 99 149 -> 94, 99 x 63 x 45 14.9 -> 14.7; single 225 x 243 x 243 120 -> 113,
+  // 225 x 243 x 105 49 -> 49 (3/2: 53), 225 x 243 x 45 26 -> 27.
   static constexpr int NROWS = 3;
   static constexpr int rows_rpb(int e) {
     if (sizeof(T) == 4) return e == 0 ? RPB : (e == 1 ? RPB / 2 * 3 : RPB / 4 * 3);
-    return e == 1 ? RPB / 2 : RPB / 4 * 3;
+    return e == 0 ? RPB : (e == 1 ? RPB / 2 : RPB / 4 * 3);
   }
   static constexpr int rows_index(int v, int nc) {
-    const int best = nc == 6 ? 0 : (sizeof(T) == 4 && FP::TPP >= 16 ? 1 : 2);
+    const int best = nc == 6 ? 0 : (sizeof(T) == 4 ? (FP::TPP >= 24 ? 1 : 2) : (FP::TPP >= 12 && FP::TPP < 16 ? 1 : 2));
     return v == 0 ? best : (v == best ? 0 : v);
   }
 };
