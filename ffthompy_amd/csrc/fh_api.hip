@@ -1914,18 +1914,17 @@ int fh_plan_create(int dim, const int* N, const double* Y, int physics, int prim
     }
     RowCfg rc32;
     row_config(pl->ax[2], pl->ncomp, sizeof(cpx<float>), (long long)pl->n0 * pl->n1, &rc32);
-    pl->rt[0] = fh::rt::make_config(sizeof(double), pl->n0, pl->n1, pl->n2, pl->ncomp);
-    pl->rt[1] = fh::rt::make_config(sizeof(float), pl->n0, pl->n1, pl->n2, pl->ncomp);
-    for (int i = 0; i < 2; ++i) {
+    const bool fixed = pl->n0 > 1 && fh::fixed_length_supported(pl->n0) && fh::fixed_length_supported(pl->n1) &&
+                       fh::fixed_length_supported(pl->n2);
+    pl->rt[0] = fh::rt::make_config(sizeof(double), pl->n0, pl->n1, pl->n2, pl->ncomp, fixed);
+    pl->rt[1] = fh::rt::make_config(sizeof(float), pl->n0, pl->n1, pl->n2, pl->ncomp, fixed);
+    for (fh::rt::Config& c : pl->rt) {
       // Where the fixed-length passes cover a 3-D grid, they stay the faster ones if the planes do not
       // fit LDS (243^3: 329 against 395 us in single, 758 against 1060 us in double precision) and for
       // double-precision planes of more than half of the LDS that need three stages an axis (125^3: 104
       // against 112 us).
-      const fh::rt::Config& c = pl->rt[i];
       const bool slow_plane = c.g.plane && c.lds > fh::rt::kLdsBytes / 2 && c.g.a2.nst > 2;
-      const bool fixed = pl->n0 > 1 && fh::fixed_length_supported(pl->n0) && fh::fixed_length_supported(pl->n1) &&
-                         fh::fixed_length_supported(pl->n2);
-      if (fixed && (!c.g.plane || slow_plane)) pl->rt[i].ok = false;
+      if (fixed && (slow_plane || (!c.g.plane && !c.thin))) c.ok = false;
     }
     pl->partial_cap = (size_t)std::max<long long>({(long long)rc.nblocks, (long long)rc32.nblocks, (long long)kScratchParts,
                                                        2LL * 36 * 1024, (long long)pl->n0 * pl->n1, 2LL * pl->rt[0].nblk,

@@ -249,6 +249,7 @@ struct ColArgs {
 // Launch shapes of one plan in one precision.
 struct Config {
   bool ok = false;
+  bool thin = false;   // rows although the planes fit: too few of them
   Geo g{};
   int nthr = 0;        // contiguous-axis passes
   unsigned nblk = 0;
@@ -343,8 +344,8 @@ bool ga_rows_config(int L, int npencils, GaRowArgs* a, int* nthr, size_t* lds);
 bool compiled_length(int L);
 
 // Shapes for a grid (3-D view n0, n1, n2; 2-D: n0 = 1) of nc components; ok = false where these passes
-// do not cover it.
-Config make_config(size_t real_bytes, int n0, int n1, int n2, int nc);
+// do not cover it. fixed: a 3-D grid that the passes of fixed lengths cover too.
+Config make_config(size_t real_bytes, int n0, int n1, int n2, int nc, bool fixed);
 
 // Stream of a launch and, if set, the events that take its start and stop times.
 struct Launch {

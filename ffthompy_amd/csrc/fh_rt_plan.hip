@@ -38,7 +38,14 @@ bool compiled_length(int L) {
   }
 }
 
-Config make_config(size_t rb, int n0, int n1, int n2, int nc) {
+// Too few planes to fill the chip, each long to transform (see make_config).
+static bool thin_planes(const Geo& g, int n1, int planes) {
+  const long long points = (long long)n1 * g.n2;
+  if (n1 == g.n2 && compiled_length(n1)) return points * (g.a2.nst > 2 ? 3 : 2) > 2 * (220LL * planes + 3300);
+  return std::min(n1, g.n2) >= 25 && planes < 128 && points > (long long)planes * planes;
+}
+
+Config make_config(size_t rb, int n0, int n1, int n2, int nc, bool fixed) {
   Config c;
   const bool three = n0 > 1;
   if (n1 < 2 || n2 < 2 || n2 > 4096 || n1 > 4096 || n0 > 4096) return c;
@@ -65,6 +72,17 @@ Config make_config(size_t rb, int n0, int n1, int n2, int nc) {
   g.plane = 0;
   if (three && div_exact((long long)(n1 + 1) * n2, n2)) set_plane(g, n1, rb, &c.nthr, &c.lds);
   if (g.plane && !(n1 == n2 && compiled_length(n2)) && n0 * nc > 256) g.plane = 0;
+  // Grids of fixed lengths have five passes with many workgroups of their own. A thin one loses by a few
+  // workgroups with a plane each and takes rows here (passes of fixed lengths / planes / rows, per application:
+  // 5 x 225 x 75 double 44 / 62 / 46 us, its 40 CG iterations 2018 / 2564 / 1771; 15 x 99 x 135 single 45 / 53 / 46;
+  // 27 x 243 x 45 single 47 / 54 / 47; 5 x 135 x 135 double 49 / 55 / 45; but 27 x 27 x 45 single 38 / 38 / 37,
+  // 15 x 99 x 99 double 49 / 48 / 49, 27 x 135 x 135 double 76 / 68 / 76, 45 x 225 x 75 double 83 / 77 / 82). The time
+  // of the planes does not depend on their number while they fit the chip, that of the rows does, hence lines
+  // between the two; 125 x 125 with its three stages costs half as much again. Planes of more than half of the LDS
+  // with three stages stay on the passes of fixed lengths (the caller's rule).
+  const bool slow = c.lds > kLdsBytes / 2 && g.a2.nst > 2;
+  c.thin = g.plane && fixed && !slow && thin_planes(g, n1, n0 * nc);
+  if (c.thin) g.plane = 0;
   if (g.plane) c.nblk = (unsigned)(n0 * nc);
   if (!g.plane) {
     // row mode: more rows per workgroup while the chip stays covered
