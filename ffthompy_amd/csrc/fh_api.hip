@@ -329,23 +329,17 @@ struct fh_batch {
   long long nvox = 0;              // voxels over all samples
   size_t lds = 0;
   fh::batch::Args args{};
+  void* mem = nullptr;             // one allocation for everything below
   fh::batch::Sample* d_smp = nullptr;
   int* d_order = nullptr;
-  int* d_counter = nullptr;
   double* d_a64 = nullptr;
   float* d_a32 = nullptr;
-  cpx<double>* d_tw64 = nullptr;
-  cpx<float>* d_tw32 = nullptr;
-  double* d_ws64 = nullptr;
-  float* d_ws32 = nullptr;
   double* d_energy = nullptr;
   int* d_kit = nullptr;
   int* d_nupd = nullptr;
   double* d_normres = nullptr;
   int* d_status = nullptr;
   fh::batch::Params* d_par = nullptr;
-  double* d_xs = nullptr;          // one load per task: solutions, then arrivals and status per load
-  int* d_pair = nullptr;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipGraph_t graph = nullptr;
@@ -2916,10 +2910,7 @@ int fh_batch_destroy(fh_batch* b) {
   if (!b) return FH_OK;
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
-  void* bufs[] = {b->d_smp, b->d_order, b->d_counter, b->d_a64, b->d_a32, b->d_tw64, b->d_tw32, b->d_ws64,
-                  b->d_ws32, b->d_energy, b->d_kit, b->d_nupd, b->d_normres, b->d_status, b->d_par, b->d_xs, b->d_pair};
-  for (void* p : bufs)
-    if (p) (void)hipFree(p);
+  if (b->mem) (void)hipFree(b->mem);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -2972,23 +2963,8 @@ int fh_batch_create(int nsamples, const int* dims, const double* Y, fh_batch** o
     return (long long)sa.n0 * sa.n1 > (long long)sc.n0 * sc.n1;
   });
   b->order_size = order;
-  const bool split = nsamples <= B::kSplitSamples;
-  if (split) {
-    // the two loads of a task follow each other
-    b->ntasks = 4 * nsamples;
-    for (std::vector<int>* o : {&b->order_sample, &b->order_size}) {
-      std::vector<int> two;
-      for (int code : *o) {
-        two.push_back(2 * code);
-        two.push_back(2 * code + 1);
-      }
-      *o = two;
-    }
-    order = b->order_size;
-  }
   int ncu = 0;
   HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, 0));
-  b->nslots = std::max(1, std::min(b->ntasks, ncu));
   // twiddle tables exp(-2 pi i m / L) of every supported length
   std::vector<cpx<double>> t64((size_t)B::NLEN * B::TWS);
   std::vector<cpx<float>> t32((size_t)B::NLEN * B::TWS);
@@ -3000,54 +2976,87 @@ int fh_batch_create(int nsamples, const int* dims, const double* Y, fh_batch** o
       t32[id * B::TWS + m] = fh::mk((float)(double)cosl(ang), (float)(double)sinl(ang));
     }
   }
-  const size_t ws64 = (size_t)b->nslots * (6 * nvec + spec64), ws32 = (size_t)b->nslots * 3 * nvec;
   hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreate(&b->ev0);
   if (e == hipSuccess) e = hipEventCreate(&b->ev1);
-  if (e == hipSuccess) e = hipMalloc(&b->d_smp, nsamples * sizeof(B::Sample));
-  if (e == hipSuccess) e = hipMalloc(&b->d_order, b->ntasks * sizeof(int));
-  if (e == hipSuccess) e = hipMalloc(&b->d_counter, 64 * sizeof(int));
-  if (e == hipSuccess) e = hipMalloc(&b->d_a64, std::max<long long>(nvox, 1) * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&b->d_a32, std::max<long long>(nvox, 1) * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&b->d_tw64, t64.size() * sizeof(cpx<double>));
-  if (e == hipSuccess) e = hipMalloc(&b->d_tw32, t32.size() * sizeof(cpx<float>));
-  if (e == hipSuccess) e = hipMalloc(&b->d_ws64, ws64 * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&b->d_ws32, ws32 * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&b->d_energy, (size_t)nsamples * 8 * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&b->d_kit, (size_t)nsamples * 4 * sizeof(int));
-  if (e == hipSuccess) e = hipMalloc(&b->d_nupd, (size_t)nsamples * 4 * sizeof(int));
-  if (e == hipSuccess) e = hipMalloc(&b->d_normres, (size_t)nsamples * 4 * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&b->d_status, (size_t)nsamples * 2 * sizeof(int));
-  if (e == hipSuccess) e = hipMalloc(&b->d_par, sizeof(B::Params));
-  if (e == hipSuccess && split) e = hipMalloc(&b->d_xs, (size_t)nsamples * 4 * nvec * sizeof(double));
-  if (e == hipSuccess && split) e = hipMalloc(&b->d_pair, (size_t)nsamples * 6 * sizeof(int));
-  if (e == hipSuccess)
-    e = hipMemcpy(b->d_smp, b->smp.data(), nsamples * sizeof(B::Sample), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(b->d_order, order.data(), b->ntasks * sizeof(int), hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(b->d_tw64, t64.data(), t64.size() * sizeof(cpx<double>), hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(b->d_tw32, t32.data(), t32.size() * sizeof(cpx<float>), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = B::allow_lds(b->lds);
   if (e != hipSuccess) return bail(fail(FH_ERR_HIP, std::string("fh_batch_create: ") + hipGetErrorString(e)));
   B::Args& A = b->args;
+  // one allocation (each costs its time, and its release more), its parts 256-byte aligned
+  auto place = [&](bool split, std::uintptr_t base) {
+    size_t at = 0;
+    auto part = [&](auto*& p, size_t count) {
+      p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + at);
+      at += (count * sizeof(*p) + 255) / 256 * 256;
+    };
+    A.split = split;
+    A.npairs = split ? 2 * nsamples : 0;
+    b->ntasks = (split ? 4 : 2) * nsamples;
+    b->nslots = std::max(1, std::min(b->ntasks, ncu));
+    A.ws64_stride = (split ? 4 : 6) * nvec + spec64;
+    A.xstride = split ? 4 * nvox : nvec;
+    A.ws32_stride = 3 * nvec;
+    cpx<double>* tw64;
+    cpx<float>* tw32;
+    part(b->d_smp, nsamples);
+    part(b->d_order, b->ntasks);
+    part(A.counter, 64);
+    part(b->d_a64, nvox);
+    part(b->d_a32, nvox);
+    part(tw64, t64.size());
+    part(tw32, t32.size());
+    part(A.ws64, (size_t)b->nslots * A.ws64_stride);
+    if (split) A.ws64 -= 2 * nvec;  // a slot starts with two solutions, which are in xs
+    part(A.ws32, (size_t)b->nslots * A.ws32_stride);
+    part(b->d_energy, (size_t)nsamples * 8);
+    part(b->d_kit, (size_t)nsamples * 4);
+    part(b->d_nupd, (size_t)nsamples * 4);
+    part(b->d_normres, (size_t)nsamples * 4);
+    part(b->d_status, (size_t)nsamples * 2);
+    part(b->d_par, 1);
+    A.tw64 = tw64;
+    A.tw32 = tw32;
+    A.xs = nullptr;
+    A.pair = A.lstat = nullptr;
+    if (split) {
+      part(A.xs, (size_t)nvox * 8);
+      part(A.pair, (size_t)nsamples * 2);
+      part(A.lstat, (size_t)nsamples * 4);
+    }
+    return at;
+  };
+  e = hipErrorOutOfMemory;
+  if (nsamples <= B::kSplitSamples) e = hipMalloc(&b->mem, place(true, 0));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    e = hipMalloc(&b->mem, place(false, 0));
+  }
+  if (e != hipSuccess) return bail(fail(FH_ERR_HIP, std::string("fh_batch_create: ") + hipGetErrorString(e)));
+  place(A.split, reinterpret_cast<std::uintptr_t>(b->mem));
+  if (A.split) {
+    // the two loads of a task follow each other
+    for (std::vector<int>* o : {&b->order_sample, &b->order_size}) {
+      std::vector<int> two;
+      for (int code : *o) {
+        two.push_back(2 * code);
+        two.push_back(2 * code + 1);
+      }
+      *o = two;
+    }
+  }
+  e = hipMemcpy(b->d_smp, b->smp.data(), nsamples * sizeof(B::Sample), hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = hipMemcpy(b->d_order, b->order_size.data(), b->ntasks * sizeof(int), hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = hipMemcpy((void*)A.tw64, t64.data(), t64.size() * sizeof(cpx<double>), hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = hipMemcpy((void*)A.tw32, t32.data(), t32.size() * sizeof(cpx<float>), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = B::allow_lds(b->lds);
+  if (e != hipSuccess) return bail(fail(FH_ERR_HIP, std::string("fh_batch_create: ") + hipGetErrorString(e)));
   A.smp = b->d_smp;
   A.order = b->d_order;
   A.ntasks = b->ntasks;
-  A.split = split;
-  A.npairs = 2 * nsamples;
-  A.xs = b->d_xs;
-  A.pair = b->d_pair;
-  A.lstat = b->d_pair ? b->d_pair + 2 * nsamples : nullptr;
-  A.counter = b->d_counter;
   A.a64 = b->d_a64;
   A.a32 = b->d_a32;
-  A.tw64 = b->d_tw64;
-  A.tw32 = b->d_tw32;
-  A.ws64 = b->d_ws64;
-  A.ws32 = b->d_ws32;
-  A.ws64_stride = 6 * nvec + spec64;
-  A.ws32_stride = 3 * nvec;
   A.nvec = nvec;
   A.energy = b->d_energy;
   A.kit = b->d_kit;

@@ -12,7 +12,7 @@ __global__ void k_batch_reset(int* counter, int* pair, int n) {
 namespace {
 
 struct Slot {
-  double *x[2], *b, *r64, *p64, *q64;
+  double *x[2], *b, *r64, *p64, *q64;  // x: only where a task is both loads (Args::split 0)
   cpx<double>* spec64;
   float *r32, *p32, *xc32;
 };
@@ -130,10 +130,10 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
     const int nv = tk.nv, N = 2 * nv;
     const double inv_n = tk.scale;
     int status = 0;
-    double* const xs0 = A.split ? A.xs + (long long)(base * 2) * A.nvec : s.x[0];  // load 1: nvec further on
+    double* const xs0 = A.split ? A.xs + 2 * sm.off + tk.pd * (A.xstride >> 1) : s.x[0];  // of load 0
 #pragma unroll 1
     for (int L = L0; L < L1; ++L) {
-      double* x = xs0 + L * A.nvec;
+      double* x = xs0 + L * A.xstride;
       CG cg;
       cg.kit = 0;
       cg.nupd = 1;
@@ -299,7 +299,7 @@ __global__ void __launch_bounds__(NT) k_batch_solve(Args A) {
       double c = a64[v];
       if (tk.pd) c = 1.0 / c;
       const double u0 = xs0[v] + 1.0, u1 = xs0[nv + v];
-      const double w0 = xs0[A.nvec + v], w1 = xs0[A.nvec + nv + v] + 1.0;
+      const double w0 = xs0[A.xstride + v], w1 = xs0[A.xstride + nv + v] + 1.0;
       dd t;
       t.lo = 0.0;
       t.hi = c * (u0 * u0 + u1 * u1);

@@ -43,9 +43,9 @@ constexpr int NT = 512;      // threads per workgroup
 constexpr int MAXL = 135;    // longest supported axis
 constexpr int TWS = 136;     // twiddle table slot (entries)
 constexpr int NLEN = 6;      // supported axis lengths
-// One load per task up to this many samples (their solutions take at most 2.4 GB): 32 samples keep 128
-// instead of 64 CUs busy (22.7 -> 11.6 ms), 512 end more evenly (45.8 -> 43.4 ms); beyond, 16 tasks and
-// more per CU balance as they are.
+// One load per task up to this many samples (their solutions, 64 bytes a voxel, have to wait for each other): 32
+// samples keep 128 instead of 64 CUs busy (22.7 -> 11.6 ms), 512 end more evenly (45.8 -> 43.4 ms); beyond, 16
+// tasks and more per CU balance as they are. Without the memory for the solutions a task is both loads too.
 constexpr int kSplitSamples = 2048;
 constexpr int kLens[NLEN] = {27, 45, 63, 81, 105, 135};
 
@@ -79,7 +79,8 @@ struct Args {
   int ntasks;
   int split;         // 1: order holds 2 (sample * 2 + pd) + load, xs the solutions, pair the arrivals
   int npairs;        // 2 * samples
-  double* xs;        // [sample][pd][load] solutions, stride nvec
+  double* xs;        // [load][pd][sample] solutions, 2 n0 n1 values each
+  long long xstride; // from a task's first solution to its second
   int* pair;         // [sample][pd] loads finished; cleared with the counter
   int* lstat;        // [sample][pd][load] status
   int* counter;      // next task; cleared by k_batch_reset before every launch
