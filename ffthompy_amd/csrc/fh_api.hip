@@ -1282,15 +1282,19 @@ constexpr double kRangeTol = 1e-12;
 
 static int solve_start(fh_plan* pl, int mode, const double* b, const double* x, bool* zero, bool* fused64) {
   const long long nv = (long long)pl->ncomp * pl->n;
-  const bool check = mode == FH_SOLVE_FP64 && rt_on<double>(pl) && pl->fused_cg && pl->op_scale == 1.0 &&
-                     pl->res_every == 0 && !pl->it_fn;
+  bool check = mode == FH_SOLVE_FP64 && rt_on<double>(pl) && pl->fused_cg && pl->op_scale == 1.0 &&
+               pl->res_every == 0 && !pl->it_fn;
+  if (check && ensure_work(pl, fused64_bytes(pl)) != FH_OK) {
+    // a coupled coefficient takes one vector more than the operator form, which may still fit
+    (void)hipGetLastError();
+    check = false;
+  }
   double* sums = pl->aux;
   int* flag = reinterpret_cast<int*>(pl->aux + 2);
   HIPCHK(hipMemsetAsync(flag, 0, sizeof(int), pl->stream));
   hipLaunchKernelGGL(fh::micro::k_count_nonzero, dim3(grid_blocks(nv, 256, 4096)), dim3(256), 0, pl->stream, nv, x,
                      flag);
   if (check) {
-    RETCHK(ensure_work(pl, fused64_bytes(pl)));
     RETCHK(rt_operator_front<double>(pl, b, fh::COEF_NONE, nullptr, nullptr));
     int nb = 0;
     RETCHK(rt_operator_back<double>(pl, nullptr, 3, b, reinterpret_cast<float*>(pl->work), pl->st, nullptr, &nb));
