@@ -822,7 +822,8 @@ class Plan:
         return ms[:nk.value].copy(), by[:nk.value].copy()
 
     def set_schedule(self, dtype, proj_variant, cols_variant, rows_variant=0):
-        """Schedule variants of the fixed-length passes for one arithmetic (fh_plan_set_schedule)."""
+        """Schedule variants of the fixed-length passes for one arithmetic (fh_plan_set_schedule; other passes
+        have none, so the operator of most grids does not depend on it)."""
         call('fh_plan_set_schedule', self._h, ctypes.c_int(dtype_code(dtype)), ctypes.c_int(int(proj_variant)),
              ctypes.c_int(int(cols_variant)), ctypes.c_int(int(rows_variant)))
 
@@ -835,8 +836,8 @@ class Plan:
     def autotune(self, dtype=np.float32, nrep=5, seed=0):
         """Time every schedule variant of the projection, strided and row passes on this plan (random
         field, 3 interleaved rounds of nrep matvecs per variant, best round; in single precision the
-        row counts on the fused CG iteration's row passes) and keep the fastest: fh_plan_autotune.
-        Returns
+        row counts on the fused CG iteration's row passes) and keep the fastest: fh_plan_autotune. Only
+        grids that run the fixed-length passes gain by it (see fh_plan_set_schedule). Returns
         {'proj_ms': [...], 'cols_ms': [...], 'rows_ms': [...], 'proj_variant': p, 'cols_variant': c,
         'rows_variant': r}."""
         dt = np.dtype(dtype)

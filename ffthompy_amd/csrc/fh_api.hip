@@ -3840,8 +3840,9 @@ int fh_potential_solve(fh_plan* pl, int mode, const double* E, double tol, int m
   pl->last_graph_batches = 0;
   // The double-precision solve runs on the passes of any smooth length (fp64 per iteration: 60 x 50 24
   // against 96 us, 128^3 116 against 480; on lengths with passes of their own 135^3 139 against 174, 81^3 54
-  // against 69, 45 x 45 24 against 33 us). Mixed precision stays on its passes: the fp32 iterations leave
-  // the potential 1e-7 to 1e-6 off inside the residual's tolerance, and that part is their rounding's.
+  // against 69, 45 x 45 24 against 33 us). Mixed precision stays on its passes, not because they are faster
+  // (100^3: 187 us an iteration on the runtime-radix kernels): the fp32 iterations leave the potential 1e-7 to
+  // 1e-6 off inside the residual's tolerance, and that part is their rounding's, so other passes move it.
   const bool rt64 = rt_on<double>(pl) && !mixed;
   const bool fused = rt64 && pl->coef_kind == fh::COEF_ISO && pl->fused_cg;
   const fh::pot::PotParams g = pot_params(pl, rt64);

@@ -349,12 +349,18 @@ int fh_last_solve_updates(const fh_plan* plan, int* n_updates);
 int fh_matvec_profile(fh_plan* plan, int dtype, const void* x, void* y, int nrep, int max_kernels,
                       double* kernel_ms, double* kernel_bytes, int* nkernels);
 
-/* Schedule of the fixed-length kernels, per arithmetic (dtype FH_F64 / FH_F32). proj_variant
+/* Schedule of the fixed-length kernels, per arithmetic (dtype FH_F64 / FH_F32). They serve the 3-D grids of fixed
+ * lengths whose planes do not fit LDS (and 125-point planes in double precision) or are ragged with
+ * n0 * ncomp > 256, and the mixed potential solves of every grid of fixed lengths. fh_matvec, fh_project, the
+ * transforms and fh_cg_solve of other plans run passes without a schedule: setting or tuning one changes nothing
+ * about them. proj_variant
  * (0..3) sets the frequency points per tile of the projection pass (forward FFT along the
- * outermost axis, G(xi), inverse FFT), which also sets the threads per workgroup; cols_variant (0..1) the columns per tile of the other strided
- * passes (3-D); rows_variant (0..2) the grid rows per workgroup of the contiguous-axis passes
- * (0, the default, the fastest on the grids measured, which depends on the axis length, the arithmetic and the
- * number of components; scalar plans, isotropic or no coefficient). Every variant computes the same values (the same
+ * outermost axis, G(xi), inverse FFT), which also sets the threads per workgroup (along 243 points 6, 4, 5, 7 in
+ * single and 3, 2, 4, 6 in double precision; more along shorter axes); cols_variant (0..1) the columns per tile of
+ * the other strided passes (3-D; 1: half as many); rows_variant (0..2) the grid rows per workgroup of the
+ * contiguous-axis passes of scalar plans with an isotropic or no coefficient: 0 the fastest of three counts for the
+ * axis and the arithmetic (8 to 32 rows by length, 3/2 of that in single or 1/2 in double precision, 3/4 of it), 1
+ * and 2 the other two. Every variant computes the same values (the same
  * transforms per pencil); only speed differs. Variant 0 is the default.
  * fh_plan_autotune times every variant on this plan (3 interleaved rounds of nrep matvecs of x
  * into y per variant, each pass timed by its own HIP events, as fh_matvec_profile; a variant's
