@@ -229,7 +229,7 @@ struct FxShape {
   // threads in 6 wavefronts, 12 rows 486 in 8, 6 rows 243 in 4, 4 rows 162 in 3) and how many workgroups
   // share a CU's LDS. Table entry 0 (RPB rows) covers every coefficient (in double precision with direct loads),
   // the others none and isotropic with 2 or 3 components, staged. rows_index: schedule variant v as a table
-  // entry; by default entry 0 with six components, else 3/4 of RPB, but 3/2 in single precision at 125, 225 and
+  // entry; by default entry 0 with six components (see rows_one_round), else 3/4 of RPB, but 3/2 in single precision at 125, 225 and
   // 243 points and half in double precision at 75 and 135. Forward + inverse rows, against RPB rows (double
   // precision: direct): double 225 x 243 x 243 326 -> 263 us, 243 x 135 x 225 195 -> 140, 225 x 243 x 135
   // 208 -> 144 (3/4: 164), 225 x 243 x 99 149 -> 94, 99 x 63 x 45 14.9 -> 14.7; single 225 x 243 x 243 120 -> 113,
@@ -238,6 +238,15 @@ struct FxShape {
   static constexpr int rows_rpb(int e) {
     if (sizeof(T) == 4) return e == 0 ? RPB : (e == 1 ? RPB / 2 * 3 : RPB / 4 * 3);
     return e == 0 ? RPB : (e == 1 ? RPB / 2 : RPB / 4 * 3);
+  }
+  // Double precision where table entry 0 runs (six components, full coefficients, single components): 3/4 of RPB,
+  // but RPB where it alone needs one round of workgroups on 256 CUs (one on a CU with six components). Elasticity,
+  // forward + inverse rows with RPB / 3/4: 45 x 45 x 225 (254 / 338 workgroups) 30.5 / 37.2 us, 45 x 81 x 135
+  // (228 / 304) 34 / 42, but 9 x 243 x 225 (274 / 365) 50.8 / 36.9, 81 x 63 x 135 (319 / 426) 56.8 / 43.4, 135 x 135 x 99
+  // 126.5 / 98.9, 45 x 225 x 243 166 / 141.
+  static constexpr bool rows_one_round(long long rows, int nc) {
+    const long long cap = 256 * (6 / nc);
+    return (rows + RPB - 1) / RPB <= cap && (rows + RPB / 4 * 3 - 1) / (RPB / 4 * 3) > cap;
   }
   static constexpr int rows_index(int v, int nc) {
     const int best = nc == 6 ? 0 : (sizeof(T) == 4 ? (FP::TPP >= 24 ? 1 : 2) : (FP::TPP >= 12 && FP::TPP < 16 ? 1 : 2));

@@ -205,6 +205,13 @@ int rows_fwd_fx_launch(const LaunchCtx& c, int nc, const T* in, const T* coef, i
                                                          partial_cap, nblocks);
     if (r != 0) return r;
   }
+  if constexpr (sizeof(T) == 8) {
+    if (!FxShape<FP, T>::rows_one_round((long long)c.n0 * c.n1, nc)) {
+      const int r = rows_fwd_fx_launch_r<T, FP, R2, true>(c, nc, in, coef, kind, out, halt, rvec, st, xc, partial,
+                                                          partial_cap, nblocks);
+      if (r != 0) return r;
+    }
+  }
   return rows_fwd_fx_launch_r<T, FP, R0, true>(c, nc, in, coef, kind, out, halt, rvec, st, xc, partial, partial_cap,
                                                nblocks);
 }
@@ -287,6 +294,13 @@ int rows_inv_fx_launch(const LaunchCtx& c, int nc, const cpx<T>* in, T* out, T s
     const int r = rows_inv_fx_launch_r<T, FP, R2, false>(c, nc, in, out, scale, epi, w, partial, partial_cap, halt,
                                                          nblocks, st);
     if (r != 0) return r;
+  }
+  if constexpr (sizeof(T) == 8) {
+    if (!FxShape<FP, T>::rows_one_round((long long)c.n0 * c.n1, nc)) {
+      const int r = rows_inv_fx_launch_r<T, FP, R2, true>(c, nc, in, out, scale, epi, w, partial, partial_cap, halt,
+                                                          nblocks, st);
+      if (r != 0) return r;
+    }
   }
   return rows_inv_fx_launch_r<T, FP, R0, true>(c, nc, in, out, scale, epi, w, partial, partial_cap, halt, nblocks, st);
 }

@@ -17,7 +17,8 @@ SCALAR = [(99, 5, 9), (99, 15, 5), (105, 9, 15), (105, 27, 25), (125, 25, 27), (
           (225, 135, 5), (243, 9, 225), (243, 5, 243), (5, 225, 243), (9, 243, 225), (15, 243, 243), (25, 225, 225),
           (27, 225, 243), (45, 225, 243), (63, 225, 225), (75, 225, 243), (81, 243, 225)]
 SIX = [(45, 9, 15), (63, 15, 9), (75, 27, 25), (81, 25, 27), (99, 5, 45), (105, 45, 5), (125, 9, 63), (135, 15, 81),
-       (225, 5, 9), (243, 9, 5), (45, 27, 99), (45, 9, 105), (45, 25, 125), (45, 15, 135), (45, 5, 225), (45, 9, 243)]
+       (225, 5, 9), (243, 9, 5), (45, 27, 99), (45, 9, 105), (45, 25, 125), (45, 15, 135), (45, 5, 225), (45, 9, 243),
+       (63, 105, 9), (45, 75, 45), (63, 27, 225)]  # the last three: one round of workgroups with more rows each
 
 
 def rel(a, b):
@@ -38,7 +39,8 @@ def plan_of(N, physics, kind, rng):
     return plan
 
 
-@pytest.mark.parametrize('physics,kind,N', [('scalar', k, N) for N in SCALAR for k in ('iso', 'full') if k == 'iso' or np.prod(N) < 4e5]
+@pytest.mark.parametrize('physics,kind,N', [('scalar', k, N) for N in SCALAR + [(99, 63, 45)] for k in ('iso', 'full')
+                                               if k == 'iso' or np.prod(N) < 4e5]
                          + [('elasticity', 'lame', N) for N in SIX] + [('elasticity', 'full', N) for N in SIX[:4]])
 def test_matvec_matches_generic_kernels(physics, kind, N):
     print('case fixed passes', physics, kind, N, flush=True)
@@ -51,6 +53,20 @@ def test_matvec_matches_generic_kernels(physics, kind, N):
         ref = plan.matvec(dx, dy).to_host()
         plan.use_generic(False)
         assert rel(plan.matvec(dx, dy).to_host(), ref) < tol, dt
+
+
+def test_transform_matches_numpy():
+    """Single components, in double precision with the larger of two row counts."""
+    N = (243, 99, 45)
+    print('case fixed transform', N, flush=True)
+    plan = nat.Plan(N, np.ones(3))
+    x = np.random.default_rng(26).standard_normal(N)
+    ref = np.fft.rfftn(x)
+    for dt, ct, tol in ((np.float64, np.complex128, 1e-12), (np.float32, np.complex64, 2e-5)):
+        X = plan.rfftn(nat.DeviceArray.from_host(x.astype(dt)[None]), nat.DeviceArray((1,) + ref.shape, ct), 1)
+        assert rel(X.to_host()[0], ref) < tol
+        z = plan.irfftn(X, nat.DeviceArray((1,) + N, dt), 1)
+        assert rel(z.to_host()[0], x) < tol
 
 
 @pytest.mark.parametrize('physics,kind,N', [('scalar', 'iso', (99, 45, 135)), ('scalar', 'iso', (105, 81, 105)),
